@@ -171,7 +171,7 @@ static lair_status getrf_impl(lair_context *ctx, int64_t m64, int64_t n64, T *a,
     // real embedding of U12 for the trailing updates is sized here, before
     // either stream of the look-ahead uses it.
     nb = std::min<int64_t>(nb, kComplexMaxNb);
-    if (kmax > 0 && rpanel_leaf_width<T>(ctx, std::max(std::min<int>((int)nb, kmax), kLeafW), m) == 0) {
+    if (kmax > 0 && rpanel_leaf_width<T>(ctx, (int)nb, m) == 0) {
       set_error("too many rows for the complex resident panel");
       return LAIR_ERR_UNSUPPORTED;
     }
@@ -210,38 +210,24 @@ static lair_status getrf_impl(lair_context *ctx, int64_t m64, int64_t n64, T *a,
   // pivots by rowmap_kernel.
   bool pmap_ok[2] = {false, false};
   auto parity = [&](int k) { return (k / (int)nb) & 1; };
-  // Leaf width of the panel at column k: the widest resident leaf, or, for
-  // FP64, half of it while at least kNarrowLeafRows rows remain.  There the
-  // FP64 bulk update (MFMA-bound) sets the pace; a leaf half as wide keeps
-  // twice the rows per workgroup, so half as many CUs are reserved for it
-  // and the bulk update gets the rest (the FP32 leaf chain is the critical
-  // path at every size, and keeps its full width).
-  constexpr int kNarrowLeafRows = 12288;
+  // Leaf width of the panel at column k (0: no resident leaf).
   auto leaf_width = [&](int k, int kb) -> int {
-    if (tournament) return 0;
-    int lw = rpanel_leaf_width<T>(ctx, kComplex ? std::max(kb, kLeafW) : kb, m - k);
-    if (std::is_same<T, double>::value && lw > kLeafW && m - k >= kNarrowLeafRows) {
-      const int lw2 = rpanel_leaf_width<T>(ctx, lw / 2, m - k);
-      if (lw2 > 0) lw = lw2;
-    }
-    return lw;
+    return tournament ? 0 : rpanel_leaf_width<T>(ctx, kb, m - k);
   };
   // Factors the panel of columns [k, k + kb) on the context's stream.
   auto factor_panel = [&](int k, int kb) -> hipError_t {
-    // Resident leaves (rows kept in LDS for the whole leaf).  A leaf narrower
-    // than the panel is followed by its interchanges on the panel's other
-    // columns, the U rows right of it (trsm) and the update below (gemm).
-    // (A complex panel narrower than the narrowest leaf goes to a leaf of
-    // that width with fewer columns.)
+    // Resident leaves.  A leaf narrower than the panel is followed by its
+    // interchanges on the panel's other columns, the U rows right of it (trsm)
+    // and the update below (gemm).
     const int lw = leaf_width(k, kb);
     const int pp = parity(k);
     pmap_ok[pp] = lw >= kb;
     if (lw > 0) {
       for (int c = k; c < k + kb; c += lw) {
         const int w = std::min(lw, k + kb - c);
-        hipError_t e2 = pmap_ok[pp] ? launch_rpanel<T>(ctx, a, lda, c, m, c, w, lw, ipiv, ctx->pmap_rows[pp],
+        hipError_t e2 = pmap_ok[pp] ? launch_rpanel<T>(ctx, a, lda, c, m, c, w, ipiv, ctx->pmap_rows[pp],
                                                        ctx->pmap_src[pp], ctx->pmap_count[pp])
-                                    : launch_rpanel<T>(ctx, a, lda, c, m, c, w, lw, ipiv);
+                                    : launch_rpanel<T>(ctx, a, lda, c, m, c, w, ipiv);
         if (e2 != hipSuccess) return e2;
         const int npv = std::min(w, m - c);
         if (npv <= 0) continue;
@@ -331,7 +317,7 @@ static lair_status getrf_impl(lair_context *ctx, int64_t m64, int64_t n64, T *a,
   auto reserve_for = [&](int k) {
     const int kb = std::min<int>((int)nb, kmax - k);
     const int lw = k < kmax ? leaf_width(k, kb) : 0;
-    ctx->panel_wgs = lw > 0 ? rpanel_grid<T>(ctx, lw, m - k) : 0;
+    ctx->panel_wgs = lw > 0 ? rpanel_grid<T>(ctx, m - k) : 0;
   };
   // Look-ahead of depth one.  Stream 1 (the context's stream) carries the
   // critical path: panel k+1's columns are updated first, then panel k+1 is
@@ -887,8 +873,7 @@ lair_status lair_context_create(lair_context **out) {
   LAIR_HIP(hipMalloc(&ctx->drec, sizeof(unsigned long long) * 2 * 64));
   LAIR_HIP(hipMalloc(&ctx->crec, sizeof(unsigned long long) * kCaluWords));
   LAIR_HIP(hipMalloc(&ctx->err, sizeof(int32_t)));
-  LAIR_HIP(hipMalloc(&ctx->rp_hdr, sizeof(unsigned long long) * kRpHdrTotal));
-  LAIR_HIP(hipMalloc(&ctx->rp_rowd, sizeof(unsigned long long) * 2 * kMaxPanelWG * kRpRowWords));
+  LAIR_HIP(hipMalloc(&ctx->rp_buf, sizeof(unsigned long long) * kRpBufWords));
   LAIR_HIP(hipMalloc(&ctx->sing, sizeof(int64_t)));
   LAIR_HIP(hipMalloc(&ctx->swap_rows, sizeof(int) * kMaxSwapRows));
   LAIR_HIP(hipMalloc(&ctx->swap_src, sizeof(int) * kMaxSwapRows));
@@ -927,9 +912,7 @@ lair_status lair_context_create(lair_context **out) {
   LAIR_HIP(launch_fill_u32(ctx.get(), reinterpret_cast<uint32_t *>(ctx->rec), 4 * kMaxPanelWG * 64, 0u));
   LAIR_HIP(launch_fill_u32(ctx.get(), reinterpret_cast<uint32_t *>(ctx->drec), 4 * 64, 0u));
   LAIR_HIP(launch_fill_u32(ctx.get(), reinterpret_cast<uint32_t *>(ctx->crec), 2 * kCaluWords, 0u));
-  LAIR_HIP(launch_fill_u32(ctx.get(), reinterpret_cast<uint32_t *>(ctx->rp_hdr), 2 * kRpHdrTotal, 0u));
-  LAIR_HIP(launch_fill_u32(ctx.get(), reinterpret_cast<uint32_t *>(ctx->rp_rowd),
-                           2 * 2 * kMaxPanelWG * kRpRowWords, 0u));
+  LAIR_HIP(launch_fill_u32(ctx.get(), reinterpret_cast<uint32_t *>(ctx->rp_buf), 2 * kRpBufWords, 0u));
   ctx->seq = 1;
   ctx->rp_seq = 1;
   if (const char *ev = std::getenv("LAIR_PANEL_MAX_WG")) ctx->rp_max_wg = std::max(1, std::atoi(ev));
@@ -947,8 +930,7 @@ lair_status lair_context_destroy(lair_context *ctx) {
   hipFree(ctx->drec);
   hipFree(ctx->crec);
   hipFree(ctx->err);
-  hipFree(ctx->rp_hdr);
-  hipFree(ctx->rp_rowd);
+  hipFree(ctx->rp_buf);
   hipFree(ctx->sing);
   hipFree(ctx->norms);
   if (ctx->pub_host) hipHostFree(ctx->pub_host);

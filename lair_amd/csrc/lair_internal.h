@@ -40,24 +40,23 @@ constexpr int kCaluWords = kCaluMaxWG * kCaluRec + kCaluDiag;
 constexpr int kReservedCUs = 32;
 // Row interchanges of one panel touch at most 2 * (panel width) rows.
 constexpr int kMaxSwapRows = 512;
-// Largest n whose row permutation is composed in LDS.
-constexpr int kPermLdsMax = 32768;
-// Tagged words per workgroup slot of the resident panel's row exchange
-// (>= leaf width * 32-bit words per element).
-constexpr int kRpRowWords = 128;
 // Columns of B per workgroup in the triangular solves with L11, and the
 // widest panel those kernels take.
 constexpr int kTrsmCW = 16;
 constexpr int kTrsmMaxKb = 128;
-// Tagged header words per workgroup slot of the resident panel's exchange:
-// real elements use 4, complex ones 1 + 2 * (32-bit words per element), in
-// slots of kRpHdrWordsMax.  The two kinds live in separate regions of the
-// header buffer (a real header's first word carries only a 16-bit tag, which
-// a complex word could match): real at 0, complex at kRpHdrComplexOff.
-constexpr int kRpHdrWords = 4;
-constexpr int kRpHdrWordsMax = 16;
-constexpr int kRpHdrComplexOff = 2 * kMaxPanelWG * kRpHdrWords;
-constexpr int kRpHdrTotal = kRpHdrComplexOff + 2 * kMaxPanelWG * kRpHdrWordsMax;  // 64-bit words
+// Resident panel leaf (rpanel.hip): widest leaf and sub-panel, and its
+// exchange buffers in tagged 64-bit words: column records (one per workgroup
+// and column parity), the pivot rows of a sub-panel (by parity) and the rows
+// that change place.
+constexpr int kRpMaxCols = 128;
+constexpr int kRpMaxW = 16;
+constexpr int kRpWaves = 4;  // waves of a leaf's workgroup, one per SIMD
+constexpr int kRpThreads = 64 * kRpWaves;
+constexpr int kRpRecWords = 64;
+constexpr int kRpRowWords = 256;  // >= leaf width * 32-bit words per element
+constexpr size_t kRpBlkOff = 2 * (size_t)kMaxPanelWG * kRpRecWords;
+constexpr size_t kRpMvOff = kRpBlkOff + 2 * (size_t)kRpMaxW * kRpRowWords;
+constexpr size_t kRpBufWords = kRpMvOff + 2 * (size_t)kRpMaxCols * kRpRowWords;
 // Widest complex panel (the triangular solve with L11 keeps L11 in LDS),
 // and the largest order of the complex getrs (unknowns of a right-hand side
 // held in registers of one 1024-thread workgroup, 16 per thread).
@@ -127,9 +126,8 @@ struct lair_context {
   // Polls a cooperative kernel's bounded wait makes before it gives up and
   // sets *err (0: every wait gives up at once).
   int32_t wait_limit = 1 << 23;
-  // Resident panel (rpanel.hip): header and row slots, tag base, grid cap.
-  unsigned long long *rp_hdr = nullptr;   // kRpHdrTotal words
-  unsigned long long *rp_rowd = nullptr;  // [2][kMaxPanelWG][kRpRowWords]
+  // Resident panel (rpanel.hip): exchange words, tag base, grid cap.
+  unsigned long long *rp_buf = nullptr;  // kRpBufWords words
   uint32_t rp_seq = 1;
   int rp_max_wg = lair::kMaxPanelWG;
   int64_t *sing = nullptr;     // last zero-pivot column (device)
@@ -223,20 +221,19 @@ template <typename T>
 hipError_t launch_panel(lair_context *ctx, T *a, int64_t lda, int row0, int m, int col0, int wcols,
                         int64_t *ipiv, int rest1, int left0);
 // Resident-panel leaf (rpanel.hip): exact partial pivoting of columns
-// [col0, col0 + wcols) over rows [row0, m), wcols <= nbw, rows kept in LDS.
+// [col0, col0 + wcols) over rows [row0, m), wcols at most the leaf width.
 // When map_rows is given, the leaf also writes the row map of its
 // interchanges (2 * npiv gather entries, see launch_rowswap_map).
 template <typename T>
 hipError_t launch_rpanel(lair_context *ctx, T *a, int64_t lda, int row0, int m, int col0, int wcols,
-                         int nbw, int64_t *ipiv, int *map_rows = nullptr, int *map_src = nullptr,
+                         int64_t *ipiv, int *map_rows = nullptr, int *map_src = nullptr,
                          int *map_count = nullptr);
-// Widest leaf width <= want (128, 64, 32 or 16) the resident panel supports
-// for `rows` rows, or 0.
+// Widest leaf <= want the resident panel supports for `rows` rows, or 0.
 template <typename T>
 int rpanel_leaf_width(lair_context *ctx, int want, int rows);
-// Workgroups of a resident leaf of width nbw over `rows` rows (0: unsupported).
+// Workgroups of a resident leaf over `rows` rows (0: unsupported).
 template <typename T>
-int rpanel_grid(lair_context *ctx, int nbw, int rows);
+int rpanel_grid(lair_context *ctx, int rows);
 // Tournament-pivoting FP32 leaf (mixed-precision factorization only).
 hipError_t launch_panel_calu(lair_context *ctx, float *a, int64_t lda, int c, int m, int wcols,
                              int64_t *ipiv, int rest1, int left0);

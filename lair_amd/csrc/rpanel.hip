@@ -1,36 +1,77 @@
-// Resident-panel LU leaf with exact partial pivoting: the column loop of
+// Panel leaf of the blocked LU with exact partial pivoting: the column loop of
 // getrf_row_major (src/lapack/getrf.rs:55-117) with iamax's choice rule
 // (src/blas/iamax.rs:6-21), for a tall leaf whose rows are spread over P
-// cooperating workgroups.
+// cooperating workgroups of R = 256 RPT rows, RPT rows per thread.
 //
-//  * Workgroup g owns R consecutive rows of the leaf.  They are loaded into
-//    LDS once and written back once, each to its final position.  Rows do not
-//    move while the leaf is factored: every row carries its current position
-//    (its row index after the interchanges so far, as the reference would
-//    see it), which is also iamax's tie-break key (lowest index wins).
-//  * One column per iteration of a runtime loop, so the code stays small
-//    enough for the instruction cache.
-//  * Per column, each workgroup publishes a header (|value|, position) for
-//    its best candidate and that candidate's row as tagged 64-bit words;
-//    every workgroup polls the P headers, picks the winner by the iamax rule
-//    and reads the winner's row.  A word is valid when its tag equals the
-//    column's tag, so no fences are needed.
-//  * The rank-1 update of pivot j (getrf.rs:76-88: l = a * (1/pivot), then
-//    a -= l * u with separate multiply and subtract) is split: column j + 1
-//    is updated at once because it decides the next pivot; the other columns
-//    are updated at the start of the next iteration while the exchange is in
-//    flight.  A published candidate row therefore still lacks the previous
-//    pivot's update beyond its pivot column.  The readers apply it with the
-//    same operands in the same order, so every copy of the pivot row is
-//    bit-identical to the owner's.
+// What bounds a leaf is the chain from one pivot to the next, so the leaf is
+// cut into sub-panels of W columns, and one column's step is as short as the
+// hardware lets it be:
+//
+//  * A row's W sub-panel entries live in registers and shift down by one each
+//    column (entry c - 1 <- entry c - l u_c, the rank-1 update of
+//    getrf.rs:76-88 with separate multiply and subtract), so every column is
+//    the same short loop body and entry 0 is always the pivot column.
+//  * Per column each wave finds its best row with 32-bit DPP maxima (the low
+//    words and positions only on ties) and its lane puts the row into LDS.
+//    With P = 1 one barrier later every thread picks the winner and updates.
+//  * With P > 1 the workgroup's best row goes out as one record of tagged
+//    64-bit words (position and the W entries, all updated), every wave polls
+//    the records of P / 4 workgroups and puts them into LDS, and one barrier
+//    later every thread picks the winner: one round trip through memory per
+//    column.  A word is valid when its tag equals the column's tag, so no
+//    fences are needed.
+//  * After a sub-panel its L is written back, the pivot rows' other columns
+//    are exchanged (one round trip per W columns), every workgroup solves
+//    U = L11^-1 A for them and updates its own rows with rank W, in place in
+//    global memory (its XCD's L2), with the same operations in the same order
+//    as the unblocked loop: a leaf's factors do not depend on W or P.  With
+//    P > 1 only the next sub-panel's columns are updated at once; the rest
+//    fills the waits of the next column loop.
+//
+// Measured per leaf, against a leaf that kept 256 rows per workgroup in LDS
+// and made two round trips per column (alone on the chip unless noted):
+// FP64, 64 columns: 70 against 165 us at 100 rows, 104 / 172 at 512, 152 /
+// 185 at 1024, 182 / 190 at 2048 inside a factorization; FP32, 128 columns:
+// 211 / 370 us at 512 rows, 346 / 385 at 1024, 369 / 397 at 4096, 411 / 435
+// at 16384.  A column costs about 0.9 us of instructions and LDS latencies
+// and, with P > 1, 0.8 us of round trip and 0.6 us for the slowest of the
+// others.
+//
+// Rows do not move while the leaf is factored: every row carries its current
+// position (its row index after the interchanges so far, as the reference
+// would see it), which is also iamax's tie-break key (lowest index wins).  At
+// the end the rows that changed place go through a tagged buffer and are
+// stored by the workgroup that owns the destination: each address of the
+// matrix is written by one workgroup only (two XCDs' L2 never hold dirty
+// bytes of the same row).
 #include <climits>
+#include <type_traits>
 
 #include "device_util.h"
 #include "lair_internal.h"
 
 namespace lair {
 
-constexpr uint32_t kRpNone = 0x1FFFFu;  // header position meaning "no candidate"
+// Sub-panel width: its record (W entries, a reciprocal and the position) is
+// one 64-bit word per lane.
+template <typename T>
+struct RpW;
+template <>
+struct RpW<float> {
+  static constexpr int W = 16;
+};
+template <>
+struct RpW<double> {
+  static constexpr int W = 16;
+};
+template <>
+struct RpW<ccplx> {
+  static constexpr int W = 16;
+};
+template <>
+struct RpW<zcplx> {
+  static constexpr int W = 8;
+};
 
 template <typename T>
 struct RpArgs {
@@ -39,85 +80,26 @@ struct RpArgs {
   int row0, m, col0, wcols, npiv, P;
   int64_t *ipiv;
   int64_t *sing;
-  unsigned long long *hdr;   // [2][kMaxPanelWG][RpHeader<T>::S] header words, by column parity
-  unsigned long long *rowd;  // [2][kMaxPanelWG][kRpRowWords] row words, by column parity
+  unsigned long long *rec;  // [2][kMaxPanelWG][kRpRecWords] column records, by column parity
+  unsigned long long *blk;  // [2][kRpMaxW][kRpRowWords] pivot rows of a sub-panel, by sub-panel parity
+  unsigned long long *mv;   // [2 * kRpMaxCols][kRpRowWords] rows that change place
   int *map_rows, *map_src, *map_count;  // row map of the leaf's interchanges (optional)
-  uint32_t seq;              // column j's tag is seq + j + 1
+  uint32_t seq;  // column j's tag is seq + j + 1, sub-panel s's seq + kRpTagBlk + s, the moves' seq + kRpTagMv
   int32_t *err;
-  int wait_limit;            // polls before a wait gives up (0: every wait gives up at once)
+  int wait_limit;  // polls before a wait gives up (0: every wait gives up at once)
 };
 
-// A candidate's header: its position, its signed pivot value v and u1, its
-// entry in the next column after every earlier pivot's update (what the
-// other workgroups need to continue before the rest of the row arrives).
-//   word 0: tag (16 bits) | position (17 bits) | high 31 bits of |v|
-//   FP32 word 1: tag (31 bits) | sign of v | bits of u1
-//   FP64 word 1: tag (32 bits) | low 32 bits of |v|
-//   FP64 word 2: tag (31 bits) | sign of v | high 32 bits of u1
-//   FP64 word 3: tag (32 bits) | low 32 bits of u1
-// S is the stride between two workgroups' headers, in words.
-template <typename T>
-struct RpHeader {
-  static constexpr int W = sizeof(T) == 8 ? 4 : 2;
-  static constexpr int S = kRpHdrWords;
-  static __device__ __forceinline__ unsigned long long word(int w, uint32_t tag, T v, T u1, int pos) {
-    const uint32_t p = pos == INT_MAX ? kRpNone : (uint32_t)pos;
-    const uint32_t sgn = v < T(0) ? 1u : 0u;
-    const T av = v < T(0) ? -v : v;
-    if constexpr (sizeof(T) == 8) {
-      const unsigned long long b = (unsigned long long)__double_as_longlong(av);
-      const unsigned long long ub = (unsigned long long)__double_as_longlong(u1);
-      if (w == 0)
-        return ((unsigned long long)(tag & 0xFFFFu) << 48) | ((unsigned long long)p << 31) |
-               ((uint32_t)(b >> 32) & 0x7FFFFFFFu);
-      if (w == 1) return tagged(tag, (uint32_t)b);
-      if (w == 2) return ((unsigned long long)(tag & 0x7FFFFFFFu) << 33) | ((unsigned long long)sgn << 32) |
-                         (uint32_t)(ub >> 32);
-      return tagged(tag, (uint32_t)ub);
-    } else {
-      if (w == 0)
-        return ((unsigned long long)(tag & 0xFFFFu) << 48) | ((unsigned long long)p << 31) |
-               (__float_as_uint(av) & 0x7FFFFFFFu);
-      return ((unsigned long long)(tag & 0x7FFFFFFFu) << 33) | ((unsigned long long)sgn << 32) |
-             __float_as_uint(u1);
-    }
-  }
-  // Tag check of word w.
-  static __device__ __forceinline__ bool ok(int w, unsigned long long x, uint32_t tag) {
-    if (w == 0) return (uint32_t)(x >> 48) == (tag & 0xFFFFu);
-    if (sizeof(T) == 4 || w == 2) return (uint32_t)(x >> 33) == (tag & 0x7FFFFFFFu);
-    return (uint32_t)(x >> 32) == tag;
-  }
-  // Position, |v| (the iamax key), v and u1 of a header whose words all
-  // carry the tag.
-  static __device__ __forceinline__ uint32_t decode(const unsigned long long *w, double &hv, T &hvs, T &hu1) {
-    const uint32_t p = (uint32_t)(w[0] >> 31) & 0x1FFFFu;
-    const uint32_t hi = (uint32_t)w[0] & 0x7FFFFFFFu;
-    uint32_t sgn;
-    if constexpr (sizeof(T) == 8) {
-      hv = __hiloint2double((int)hi, (int)(uint32_t)w[1]);
-      sgn = (uint32_t)(w[2] >> 32) & 1u;
-      hu1 = __hiloint2double((int)(uint32_t)w[2], (int)(uint32_t)w[3]);
-    } else {
-      hv = (double)__uint_as_float(hi);
-      sgn = (uint32_t)(w[1] >> 32) & 1u;
-      hu1 = __uint_as_float((uint32_t)w[1]);
-    }
-    hvs = sgn ? -(T)hv : (T)hv;
-    return p;
-  }
-};
+constexpr uint32_t kRpTagBlk = 160, kRpTagMv = 192, kRpTags = 256;
+static_assert(kRpMaxCols < (int)kRpTagBlk && kRpTagBlk + kRpMaxCols / 8 < kRpTagMv, "tags of a launch are distinct");
 
 // iamax's key (src/blas/iamax.rs:14: |re| + |im| in the real type) and the
 // pivot reciprocal (getrf.rs:76) of a real or complex element.
 template <typename T>
-__device__ __forceinline__ double rp_key(T x) {
-  if constexpr (cplx_traits<T>::is) {
-    const typename cplx_traits<T>::real k = fabs(x.re) + fabs(x.im);
-    return (double)k;
-  } else {
-    return fabs((double)x);
-  }
+__device__ __forceinline__ typename cplx_traits<T>::real rp_key(T x) {
+  if constexpr (cplx_traits<T>::is)
+    return fabs(x.re) + fabs(x.im);
+  else
+    return fabs(x);
 }
 template <typename T>
 __device__ __forceinline__ T rp_recip(T v) {
@@ -127,521 +109,931 @@ __device__ __forceinline__ T rp_recip(T v) {
     return T(1) / v;
 }
 
-// Complex header: the key is recomputed from v by every reader, so the
-// header carries the position and the full values of v and u1, each 32-bit
-// part under a 32-bit tag.
-//   word 0: tag | position; words 1..H: v; words H+1..2H: u1
+// Maximum of unsigned words over the wave (ROWS = 4) or over each row of 16
+// lanes (ROWS = 1), in every lane.
+template <int ROWS>
+__device__ __forceinline__ uint32_t lanes_max_u32(uint32_t x) {
+  auto step = [](uint32_t v, uint32_t o) { return v > o ? v : o; };
+  x = step(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, true));
+  x = step(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, true));
+  x = step(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x141, 0xF, 0xF, true));
+  x = step(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x140, 0xF, 0xF, true));
+  if constexpr (ROWS == 4) {
+    const auto p = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    x = step(p[0], p[1]);
+    const auto q = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    x = step(q[0], q[1]);
+  }
+  return x;
+}
+
+// iamax over one wave: the lane whose key is largest and, among equal keys,
+// whose position is lowest; -1 without a candidate (key > 0, so zero and NaN
+// are never chosen).  Keys are non-negative, so their bit patterns order as
+// unsigned words.
 template <typename R>
-struct RpHeader<cplx<R>> {
-  typedef cplx<R> T;
-  static constexpr int H = sizeof(T) / 4;
-  static constexpr int W = 1 + 2 * H;
-  static constexpr int S = kRpHdrWordsMax;
-  static __device__ __forceinline__ unsigned long long word(int w, uint32_t tag, T v, T u1, int pos) {
-    const uint32_t p = pos == INT_MAX ? kRpNone : (uint32_t)pos;
-    if (w == 0) return tagged(tag, p);
-    return tagged(tag, w <= H ? word_of<T>(v, w - 1) : word_of<T>(u1, w - 1 - H));
+__device__ __forceinline__ int wave_best(R key, int pos) {
+  const bool cand = key > R(0);
+  if (!__builtin_amdgcn_ballot_w64(cand)) return -1;
+  uint32_t kh, kl = 0;
+  if constexpr (sizeof(R) == 8) {
+    kh = (uint32_t)__double2hiint(key);
+    kl = (uint32_t)__double2loint(key);
+  } else {
+    kh = __float_as_uint(key);
   }
-  static __device__ __forceinline__ bool ok(int, unsigned long long x, uint32_t tag) {
-    return (uint32_t)(x >> 32) == tag;
+  const uint32_t mh = lanes_max_u32<4>(cand ? kh : 0u);
+  bool in = cand && kh == mh;
+  if constexpr (sizeof(R) == 8) {
+    const uint32_t ml = lanes_max_u32<4>(in ? kl : 0u);
+    in = in && kl == ml;
   }
-  static __device__ __forceinline__ uint32_t decode(const unsigned long long *w, double &hv, T &hvs, T &hu1) {
-    uint32_t a[H], b[H];
-#pragma unroll
-    for (int k = 0; k < H; ++k) {
-      a[k] = (uint32_t)w[1 + k];
-      b[k] = (uint32_t)w[1 + H + k];
-    }
-    hvs = from_words<T>(a);
-    hu1 = from_words<T>(b);
-    hv = rp_key(hvs);
-    return (uint32_t)w[0];
+  const uint32_t mp = lanes_max_u32<4>(in ? ~(uint32_t)pos : 0u);
+  const unsigned long long b = __builtin_amdgcn_ballot_w64(in && ~(uint32_t)pos == mp);
+  return __ffsll((long long)b) - 1;
+}
+
+// The high word of an element's key, which alone decides a comparison unless
+// two are equal or one is zero, subnormal, infinite or NaN: a maximum in
+// [1, kKeyTop) with one holder is iamax's choice, anything else goes through
+// wave_best.
+template <typename T>
+__device__ __forceinline__ uint32_t key_hi(T x) {
+  typedef typename cplx_traits<T>::real R;
+  R k;
+  if constexpr (cplx_traits<T>::is)
+    k = fabs(x.re) + fabs(x.im);
+  else
+    k = x;
+  if constexpr (sizeof(R) == 8)
+    return (uint32_t)__double2hiint(k);
+  else
+    return __float_as_uint(k);
+}
+template <typename R>
+constexpr uint32_t kKeyTop = sizeof(R) == 8 ? 0x7FF00000u : 0x7F800000u;
+// Whether a maximum needs wave_best (uniform).
+template <typename R>
+__device__ __forceinline__ bool key_rare(uint32_t mh, int holders) {
+  const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane((int)mh);
+  return holders != 1 || m - 1u >= kKeyTop<R> - 1u;
+}
+
+// Values computed here, not later under a branch.
+template <typename T>
+__device__ __forceinline__ void pin(T &x) {
+  if constexpr (cplx_traits<T>::is) {
+    __asm__ volatile("" : "+v"(x.re), "+v"(x.im));
+  } else {
+    __asm__ volatile("" : "+v"(x));
   }
+}
+
+template <typename T>
+__device__ __forceinline__ T sel(bool c, T x, T y) {
+  if constexpr (cplx_traits<T>::is)
+    return T(c ? x.re : y.re, c ? x.im : y.im);
+  else
+    return c ? x : y;
+}
+
+// N elements from 16-byte aligned LDS, by 16-byte reads.
+template <typename T, int N>
+__device__ __forceinline__ void lds_get(T (&x)[N], const T *src) {
+  __builtin_memcpy(x, __builtin_assume_aligned(src, 16), sizeof(T) * N);
+}
+
+// Sizes of the kernel's LDS regions.
+template <typename T, int RPT, int MR>
+struct RpLds {
+  typedef typename cplx_traits<T>::real R;
+  static constexpr int W = RpW<T>::W;
+  static constexpr int WPE = sizeof(T) / 4;
+  // A record in 32-bit words: W entries, the position, the row it was loaded
+  // from; RW is its pitch in LDS, with a spare word NW that the lanes past it
+  // write.
+  static constexpr int EW = W * WPE, PW = EW, OW = PW + 1, NW = OW + 1;
+  static constexpr int RW = (NW + 4) & ~3;
+  static constexpr int NR = kRpThreads * RPT;
+  // Column pitch of the L tile: 16-byte aligned quads of rows, and the
+  // coalesced loads (W lanes to a row) spread over all banks.
+  static constexpr int LP = NR + (sizeof(T) == 4 ? 4 : 2);
+  static constexpr int NBM = sizeof(T) == 4 ? kRpMaxCols : 64;  // widest leaf
+  static constexpr int RESTM = NBM - W;
+  static constexpr int MOVED = 2 * NBM < NR ? 2 * NBM : NR;  // rows of a workgroup that change place, at most
+  // The update of the columns beyond the next sub-panel is put off into the
+  // next column loop's waits (needs two L tiles).
+  static constexpr bool kDefer = MR > 0 && RPT <= 2;
+  static constexpr size_t kTile = sizeof(T) * W * LP;
+  static constexpr size_t kL = (kDefer ? 2 : 1) * kTile;
+  static constexpr size_t kC = sizeof(uint32_t) * 2 * kRpWaves * RW;
+  static constexpr size_t kU11 = sizeof(T) * W * W;
+  static constexpr size_t kRec = sizeof(uint32_t) * 2 * (MR * kRpWaves) * RW;
+  static constexpr size_t kLL = sizeof(T) * W * W;
+  static constexpr size_t kU = sizeof(T) * (size_t)W * RESTM;
+  static constexpr size_t kRecLL = kRec > kLL ? kRec : kLL;
+  static constexpr size_t total = kL + kC + kU11 + kRecLL + kU;
+  static_assert(3 * sizeof(int) * MOVED <= kTile, "the lists of moved rows take the tile's place");
 };
 
-// Waves: wave 0 communicates (publishes, polls, rebuilds pivot rows) and
-// owns no rows; waves 1..NWK own RPT rows per lane, R = 64 * NWK * RPT rows.
-template <typename T, int NB, int NWK, int RPT>
-__global__ void __launch_bounds__(64 * (NWK + 1)) rpanel_kernel(RpArgs<T> pa) {
+// RPT: rows per thread.  MR: workgroup records each wave polls (P <= MR *
+// kRpWaves); 0: P = 1.
+//
+// A column costs its instructions (every wave's, four cycles each) plus a few
+// LDS and memory latencies, so a workgroup is one wave per SIMD whatever its
+// rows, and the column loop is written without branches where the hardware
+// allows it (a taken branch costs as much as eight vector instructions):
+// loads are clamped rather than masked, every row computes, and what a
+// retired row computes is not used.
+template <typename T, int RPT, int MR>
+__global__ void __launch_bounds__(kRpThreads) rpanel_kernel(RpArgs<T> pa) {
 #pragma clang fp contract(off)
-  constexpr int NT = 64 * (NWK + 1);
-  constexpr int NW = 64 * NWK;  // worker threads
-  constexpr int R = NW * RPT;
-  // Column-major tile with a padded column: a worker's sweep along its row
-  // and a wave's copy of one row (lanes along the columns) are both free of
-  // bank conflicts.
-  constexpr int LDC = R + 1;
-  constexpr int WPE = sizeof(T) / 4;
-  constexpr int NI = (NB + 63) / 64;
-  constexpr int HW = RpHeader<T>::W;
-  static_assert(NB * WPE <= kRpRowWords && HW <= RpHeader<T>::S, "exchange record sizes");
+  constexpr bool MULTI = MR > 0;
+  typedef RpLds<T, RPT, MR> S;
+  typedef typename S::R R;
+  constexpr int W = S::W, WPE = S::WPE, EW = S::EW, PW = S::PW, OW = S::OW, NW = S::NW, RW = S::RW, LP = S::LP,
+                NR = S::NR, NWV = kRpWaves, NT = kRpThreads;
+  constexpr int WR = 64 * RPT;  // rows of a wave
+  constexpr int RS = 64 / W;    // rows a wave copies at a time (W lanes to a row)
+  typedef uint32_t raw_t __attribute__((ext_vector_type(WPE)));  // an element, for copies
+  constexpr int JW = W / NWV;   // pivot rows of a sub-panel per wave
+  static_assert(NW < 64 && kRpRecWords >= 64, "a record is one word per lane");
+  static_assert(W <= kRpMaxW && S::NBM * WPE <= kRpRowWords, "exchanged rows fit their slots");
+  static_assert(W * W <= NT && S::RESTM <= 2 * 64 && W % NWV == 0, "one pass over L11, two over a pivot row");
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  T *s_a = reinterpret_cast<T *>(smem_raw);  // [NB][LDC] the workgroup's rows, by column
-  __shared__ T s_wrow[2][NWK][NB];           // worker waves' best rows (columns j-1..)
-  __shared__ T s_u[2][NB];                   // pivot rows
-  __shared__ double s_wv[2][NWK];
-  __shared__ int s_wp[2][NWK];
-  __shared__ T s_recip[2], s_u1[2];
-  __shared__ int s_at[NB];  // original row now at position row0 + e
-  __shared__ int s_pw[2], s_occ[2], s_none[2], s_q[2];
-  __shared__ int s_fin[R];  // final positions for the write-back
-  __shared__ int s_bail;
+  T *s_l = reinterpret_cast<T *>(smem_raw);                                // [W][LP] sub-panel, by column
+  T *s_lold = reinterpret_cast<T *>(smem_raw + S::kL - S::kTile);          // the one before (kDefer)
+  uint32_t *s_c = reinterpret_cast<uint32_t *>(smem_raw + S::kL);          // [2][NWV][RW] waves' best rows
+  T *s_u11 = reinterpret_cast<T *>(smem_raw + S::kL + S::kC);              // [W][W] pivot rows, from their pivots on
+  unsigned char *un_raw = smem_raw + S::kL + S::kC + S::kU11;
+  uint32_t *s_r = reinterpret_cast<uint32_t *>(un_raw);                    // [2][MR * NWV][RW] workgroups' records
+  T *s_lt = reinterpret_cast<T *>(un_raw);                                 // [W][W] L11 (between the column loops)
+  T *s_u = reinterpret_cast<T *>(un_raw + S::kRecLL);                      // [W][un] pivot rows, then U
+  __shared__ int s_po[kRpMaxCols];  // rows that the pivot rows were loaded from
+  __shared__ __align__(16) int s_pw[kRpMaxCols];  // pivot positions of the leaf
+  __shared__ int s_cnt, s_bail;
 
-  const int g = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int tw = t - 64;  // worker index (rows tw + s * NW)
-  const int base = pa.row0 + g * R;
+  const int g = blockIdx.x, t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int base = pa.row0 + g * NR;
+  const int nvalid = min(NR, pa.m - base);  // rows of this workgroup
   const int ncols = pa.wcols;
+  T *const rows = pa.a + (int64_t)base * pa.lda + pa.col0;  // this workgroup's rows of the leaf
+  T *const wrows = rows + (int64_t)(wave * WR) * pa.lda;    // this wave's rows
+  const int r0 = wave * WR + lane;                          // this thread's first row (the others 64 apart)
 
-  // Load: wave w copies rows w, w + NWK + 1, ... (coalesced along the row).
-  for (int i = wave; i < R; i += NWK + 1) {
-    const int r = base + i;
-    const bool okr = r < pa.m;
-    const T *src = pa.a + (int64_t)(okr ? r : 0) * pa.lda + pa.col0;
-#pragma unroll
-    for (int q = 0; q < NI; ++q) {
-      const int c = lane + 64 * q;
-      if (c < NB) s_a[c * LDC + i] = (okr && c < ncols) ? src[c] : T(0);
-    }
-  }
   int cpos[RPT];
-  bool act[RPT];
-  T lr[RPT];
-  // Entry j of each row (all updates through pivot j - 1) and entry j + 1
-  // after the pending update, kept in registers between the phases that
-  // produce and use them.
-  T cj[RPT], c1[RPT];
+  uint32_t amask[RPT];  // sign-clearing mask while the row is a candidate, else zero
 #pragma unroll
   for (int s = 0; s < RPT; ++s) {
-    cpos[s] = base + tw + s * NW;
-    act[s] = wave > 0 && cpos[s] < pa.m;
-    lr[s] = T(0);
+    cpos[s] = base + r0 + 64 * s;
+    amask[s] = r0 + 64 * s < nvalid ? 0x7FFFFFFFu : 0u;
   }
-  for (int e = t; e < NB; e += NT) s_at[e] = pa.row0 + e;
-  if (t == 0) s_bail = 0;
-  __syncthreads();
-#pragma unroll
-  for (int s = 0; s < RPT; ++s) {
-    cj[s] = wave > 0 ? s_a[tw + s * NW] : T(0);
-    c1[s] = T(0);
-  }
-
-  bool pend = false;  // the previous pivot's update of columns > j is pending
-  // Wave 0: the winning row's entries j + 1 .. NB - 1 and its multiplier
-  // entry j - 1 (tagged words; columns past the row read as valid zeros).
-  unsigned long long rw[NI][WPE], mw[WPE];
-  auto load_row = [&](int q, int jj, uint32_t tag, bool pnd) {
-    const unsigned long long *rs = pa.rowd + ((size_t)(jj & 1) * kMaxPanelWG + q) * kRpRowWords;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int c = jj + 1 + lane + 64 * i;
-#pragma unroll
-      for (int p = 0; p < WPE; ++p) rw[i][p] = c < NB ? ld_agent(rs + c * WPE + p) : tagged(tag, 0);
-    }
-#pragma unroll
-    for (int p = 0; p < WPE; ++p) mw[p] = pnd ? ld_agent(rs + (jj - 1) * WPE + p) : tagged(tag, 0);
-  };
-  int j = 0;
-  for (; j < pa.npiv; ++j) {
-    const int par = j & 1;
-    const int d = pa.row0 + j;
-    const uint32_t tg = pa.seq + (uint32_t)j + 1u;
-
-    if (wave > 0) {
-      // W1. Candidates of column j: |a| > 0, largest first, lowest position
-      //     on ties; the wave's best row is copied (from column j - 1, the
-      //     multiplier of the pending update) before that update changes it.
-      double bv = 0.0;
-      int bp = INT_MAX, bs = -1;
-#pragma unroll
-      for (int s = 0; s < RPT; ++s) {
-        if (act[s]) {
-          const double x = rp_key(cj[s]);
-          if (x > bv || (x == bv && x > 0.0 && cpos[s] < bp)) {
-            bv = x;
-            bp = cpos[s];
-            bs = s;
-          }
-        }
-      }
-      double wv;
-      int wp;
-      wave_argmax(bv, bp, wv, wp);
-      if (wp != INT_MAX) {
-        const unsigned long long hit = __ballot(bs >= 0 && bp == wp);
-        const int wl = __ffsll((long long)hit) - 1;
-        const int wsel = __builtin_amdgcn_readlane(bs, wl);
-        const int li = (wave - 1) * 64 + wl + wsel * NW;
-        for (int c = (j > 0 ? j - 1 : 0) + lane; c < NB; c += 64) s_wrow[par][wave - 1][c] = s_a[c * LDC + li];
-      }
-      if (lane == 0) {
-        s_wv[par][wave - 1] = wv;
-        s_wp[par][wave - 1] = wp;
-      }
-    }
-    __syncthreads();  // B1
-
-    if (wave == 0) {
-      // C2. The workgroup's candidate, its header and its row.
-      double cv = s_wv[par][0];
-      int cp = s_wp[par][0], cw = 0;
-#pragma unroll
-      for (int q = 1; q < NWK; ++q) {
-        const double ov = s_wv[par][q];
-        const int op = s_wp[par][q];
-        if (ov > cv || (ov == cv && op < cp)) {
-          cv = ov;
-          cp = op;
-          cw = q;
-        }
-      }
-      T cvs = T(0), cu1 = T(0);
-      if (cp != INT_MAX) {
-        const T *wr = s_wrow[par][cw];
-        cvs = wr[j];
-        if (j + 1 < NB) {
-          cu1 = wr[j + 1];
-          if (pend) {
-            const T e = wr[j - 1] * s_u[par ^ 1][j + 1];
-            cu1 = cu1 - e;
-          }
-        }
-      }
-      unsigned long long *hs = pa.hdr + ((size_t)par * kMaxPanelWG + g) * RpHeader<T>::S;
-      if (lane < HW) st_agent(hs + lane, RpHeader<T>::word(lane, tg, cvs, cu1, cp));
-      if (cp != INT_MAX) {
-        unsigned long long *rs = pa.rowd + ((size_t)par * kMaxPanelWG + g) * kRpRowWords;
-        for (int idx = (j > 0 ? j - 1 : 0) * WPE + lane; idx < NB * WPE; idx += 64)
-          st_agent(rs + idx, tagged(tg, word_of<T>(s_wrow[par][cw][idx / WPE], idx % WPE)));
-      }
-
-      // C3. All headers; the winner by the iamax rule.
-      bool bail = false;
-      double hv = 0.0;
-      int hp = INT_MAX;
-      T hvs = T(0), hu1 = T(0);
-      {
-        const unsigned long long *hb = pa.hdr + (size_t)par * kMaxPanelWG * RpHeader<T>::S;
-        int spins = 0;
-        for (;;) {
-          if (spins >= pa.wait_limit) {
-            bail = true;
-            break;
-          }
-          bool ok = true;
-          if (lane < pa.P) {
-            unsigned long long w[HW];
-#pragma unroll
-            for (int k = 0; k < HW; ++k) {
-              w[k] = ld_agent(hb + lane * RpHeader<T>::S + k);
-              ok = ok && RpHeader<T>::ok(k, w[k], tg);
-            }
-            const uint32_t p = RpHeader<T>::decode(w, hv, hvs, hu1);
-            hp = p == kRpNone ? INT_MAX : (int)p;
-            if (hp == INT_MAX) hv = 0.0;
-          }
-          if (__all(ok)) break;
-          if ((++spins & 63) == 0 && ld_agent(pa.err) != 0) {
-            bail = true;
-            break;
-          }
-        }
-      }
-      double gv;
-      int gp;
-      wave_argmax(hv, hp, gv, gp);
-      const bool none = gp == INT_MAX;
-      // C4. The winner's row loads are issued now and stay in flight
-      //     through the bookkeeping and the barrier (C5 completes them).
-      int q = 0;
-      if (!none && !bail) {
-        q = __ffsll((long long)__ballot(lane < pa.P && hp == gp)) - 1;
-        load_row(q, j, tg, pend);
-      }
-      if (lane == 0) {
-        const int occ = s_at[j];
-        const int pw = none ? d : gp;
-        s_pw[par] = pw;
-        s_occ[par] = occ;
-        s_none[par] = none ? 1 : 0;
-        if (pw != d && pw - pa.row0 < NB) s_at[pw - pa.row0] = occ;
-        if (g == 0 && !bail) {
-          pa.ipiv[d] = pw;
-          if (none) *pa.sing = d;
-        }
-        if (bail) {
-          s_bail = 1;
-          atomic_or_agent(pa.err, kErrWait);
-        }
-      }
-      if (!none) {
-        const T v = readlane_t(hvs, q), u1 = readlane_t(hu1, q);
-        if (lane == 0) {
-          s_recip[par] = rp_recip(v);
-          s_u1[par] = u1;
-          s_q[par] = q;
-          s_u[par][j] = v;
-        }
-      }
-    } else if (pend) {
-      // W3. The pending update of columns > j with the previous pivot row,
-      //     while wave 0 exchanges; eight columns in flight at a time.
-      const T *u = s_u[par ^ 1];
-#pragma unroll
-      for (int s = 0; s < RPT; ++s) {
-        if (act[s]) {
-          T *row = s_a + tw + s * NW;
-          const T l = lr[s];
-          int c = j + 1;
-          if (c < ncols) {
-            const T e = l * u[c];
-            c1[s] = row[c * LDC] - e;
-            row[c * LDC] = c1[s];
-            ++c;
-          }
-          for (; c + 8 <= ncols; c += 8) {
-            T x[8], y[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-              x[q] = row[(c + q) * LDC];
-              y[q] = u[c + q];
-            }
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-              const T e = l * y[q];
-              row[(c + q) * LDC] = x[q] - e;
-            }
-          }
-          for (; c < ncols; ++c) {
-            const T e = l * u[c];
-            row[c * LDC] = row[c * LDC] - e;
-          }
-        }
-      }
-    }
-    __syncthreads();  // B2
-    if (s_bail) break;
-    const bool none = s_none[par] != 0;
-
-    if (wave == 0) {
-      // C5. The winner's full row, rebuilt as its owner holds it after the
-      //     pending update (same operands, same order), for the next
-      //     iteration's update; read while the workers go on.
-      if (!none) {
-        bool bail = false;
-        int spins = 0;
-        for (;;) {
-          bool ok = true;
-#pragma unroll
-          for (int i = 0; i < NI; ++i)
-#pragma unroll
-            for (int p = 0; p < WPE; ++p) ok = ok && (uint32_t)(rw[i][p] >> 32) == tg;
-#pragma unroll
-          for (int p = 0; p < WPE; ++p) ok = ok && (uint32_t)(mw[p] >> 32) == tg;
-          if (__all(ok)) break;
-          if (spins >= pa.wait_limit || ((++spins & 63) == 0 && ld_agent(pa.err) != 0)) {
-            bail = true;
-            break;
-          }
-          load_row(s_q[par], j, tg, pend);
-        }
-        T rv[NI];
-        T mult = T(0);
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          uint32_t w[WPE];
-#pragma unroll
-          for (int p = 0; p < WPE; ++p) w[p] = (uint32_t)rw[i][p];
-          rv[i] = from_words<T>(w);
-        }
-        if (pend) {
-          uint32_t w[WPE];
-#pragma unroll
-          for (int p = 0; p < WPE; ++p) w[p] = (uint32_t)mw[p];
-          mult = from_words<T>(w);
-        }
-        if (bail) {
-          // The status word is set, so the next exchange gives up at once
-          // and the loop ends at the next barrier.
-          if (lane == 0) {
-            s_bail = 1;
-            atomic_or_agent(pa.err, kErrWait);
-          }
-        } else {
-#pragma unroll
-          for (int i = 0; i < NI; ++i) {
-            const int c = j + 1 + lane + 64 * i;
-            if (c < NB) {
-              T u = rv[i];
-              if (pend) {
-                const T e = mult * s_u[par ^ 1][c];
-                u = u - e;
-              }
-              s_u[par][c] = u;
-            }
-          }
-        }
-      }
-    } else {
-      // W5. Interchange bookkeeping (the pivot row takes position d, the row
-      //     at d takes the pivot's old position), then the multipliers of
-      //     column j and the update of column j + 1.  A column without a
-      //     nonzero candidate is left unscaled (getrf.rs:72-73).
-      const int pw = s_pw[par], occ = s_occ[par];
-#pragma unroll
-      for (int s = 0; s < RPT; ++s) {
-        if (act[s] && cpos[s] == pw) {
-          act[s] = false;
-          cpos[s] = d;
-        } else if (base + tw + s * NW == occ) {
-          cpos[s] = pw;
-        }
-      }
-      const T recip = s_recip[par], u1 = s_u1[par];
-#pragma unroll
-      for (int s = 0; s < RPT; ++s) {
-        if (act[s]) {
-          T *row = s_a + tw + s * NW;
-          const T v1 = (j + 1 < ncols) ? (pend ? c1[s] : row[(j + 1) * LDC]) : T(0);
-          if (!none) {
-            const T l = cj[s] * recip;
-            row[j * LDC] = l;
-            lr[s] = l;
-            if (j + 1 < ncols) {
-              const T e = l * u1;
-              cj[s] = v1 - e;
-              row[(j + 1) * LDC] = cj[s];
-            }
-          } else {
-            cj[s] = v1;
-          }
-        }
-      }
-    }
-    pend = !none;
+  // Record keys of the waves and, in lanes, of the workgroups.
+  const uint32_t wmask = lane < NWV ? 0x7FFFFFFFu : 0u, pmask = lane < pa.P ? 0x7FFFFFFFu : 0u;
+  for (int e = t; e < kRpMaxCols; e += NT) s_po[e] = -1;
+  if (t == 0) {
+    s_bail = pa.wait_limit <= 0 ? 1 : 0;
+    s_cnt = 0;
   }
   __syncthreads();
-  if (s_bail) {
-    // Given up: identity pivots for the columns not decided keep the
-    // interchanges queued after this launch in bounds (thread 0 of workgroup
-    // 0 writes every pivot of the leaf).
-    if (g == 0 && t == 0) {
-      for (int jj = j; jj < pa.npiv; ++jj) pa.ipiv[pa.row0 + jj] = pa.row0 + jj;
-      if (pa.map_count) *pa.map_count = 0;
-    }
-    return;
-  }
+  bool bail = s_bail != 0;
+  if (bail && t == 0) atomic_or_agent(pa.err, kErrWait);
+  int done = 0;         // pivots decided
+  int last_none = -1;  // last column without a candidate
 
-  // The last pivot's update of the columns beyond the pivots (wide leaves).
-  if (pend && wave > 0) {
-    const int jl = pa.npiv - 1;
+  // The first sub-panel (each wave its own rows, W lanes to a row); the later
+  // ones come from the update before them.
+  {
+    const int wc = lane % W, wr = lane / W, cw = min(W, ncols);
+    const T *src = wrows + (int64_t)wr * pa.lda + wc;
 #pragma unroll
     for (int s = 0; s < RPT; ++s) {
-      if (act[s]) {
-        T *row = s_a + tw + s * NW;
-        for (int c = jl + 2; c < ncols; ++c) {
-          const T e = lr[s] * s_u[jl & 1][c];
-          row[c * LDC] = row[c * LDC] - e;
-        }
-      }
+      T x[W];
+#pragma unroll
+      for (int i = 0; i < W; ++i)
+        x[i] = wave * WR + 64 * s + wr + i * RS < nvalid && wc < cw ? src[(int64_t)(64 * s + i * RS) * pa.lda] : T(0);
+#pragma unroll
+      for (int i = 0; i < W; ++i) s_l[wc * LP + wave * WR + 64 * s + wr + i * RS] = x[i];
     }
   }
+
+  // One block of the update A22 -= L21 U after a sub-panel that ended at
+  // column c1: 64 of this wave's rows by W columns, separate multiply and
+  // subtract, the columns of L in order: the same operations, in the same
+  // order, as the unblocked column loop.  Each lane keeps 4 rows by TC
+  // columns, so 16 bytes read from LDS feed four products.
+  constexpr int TC = W / 4;
+  struct Upd {
+    int c1 = 0, rest = 0, un = 0, next = -1;  // next block (its rows vary fastest), counting down
+    const T *l = nullptr;
+    unsigned long long live[RPT] = {};
+  } upd;
+  const int rg = (lane >> 2) * 4, cg = (lane & 3) * TC;
+  auto upd_live = [&](int rb) {
+    unsigned long long m = upd.live[0];
+#pragma unroll
+    for (int s = 1; s < RPT; ++s) m = rb == s ? upd.live[s] : m;
+    return (unsigned)(m >> rg) & 15u;
+  };
+  // C of block idx (whole: all its columns lie in the leaf).  Rows that do
+  // not live load from a valid place and are not stored.
+  auto upd_fetch = [&](int idx, T (&x)[4][TC]) {
+    const int rb = idx % RPT, n0 = idx / RPT * W;
+    const unsigned live = upd_live(rb);
+    const T *cb = wrows + (int64_t)(64 * rb + rg) * pa.lda + upd.c1 + n0 + cg, *safe = rows + upd.c1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) __builtin_memcpy(x[i], live >> i & 1u ? cb + i * pa.lda : safe, sizeof(T) * TC);
+  };
+  auto upd_fetch_edge = [&](int idx, T (&x)[4][TC]) {
+    const int rb = idx % RPT, n0 = idx / RPT * W;
+    const unsigned live = upd_live(rb);
+    const T *cb = wrows + (int64_t)(64 * rb + rg) * pa.lda + upd.c1, *safe = rows + upd.c1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int q = 0; q < TC; ++q)
+        x[i][q] = (live >> i & 1u ? cb + i * pa.lda : safe)[min(n0 + cg + q, upd.rest - 1)];
+  };
+  auto upd_mul_part = [&](int idx, T (&x)[4][TC], auto k0_, auto k1_) {
+    constexpr int k0 = decltype(k0_)::value, k1 = decltype(k1_)::value;
+    const int rb = idx % RPT, n0 = idx / RPT * W;
+    const T *ucol = s_u + min(n0 + cg, upd.un - TC) + k0 * upd.un, *lcol = upd.l + wave * WR + 64 * rb + rg;
+    T u[2][TC], l[2][4];
+    lds_get<T, TC>(u[0], ucol);
+    lds_get<T, 4>(l[0], lcol + k0 * LP);
+#pragma unroll
+    for (int k = k0; k < k1; ++k) {
+      const int b = (k - k0) & 1;
+      if (k + 1 < k1) {
+        ucol += upd.un;
+        lds_get<T, TC>(u[b ^ 1], ucol);
+        lds_get<T, 4>(l[b ^ 1], lcol + (k + 1) * LP);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // the next operands are on their way
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int q = 0; q < TC; ++q) {
+          const T e = l[b][i] * u[b][q];
+          x[i][q] = x[i][q] - e;
+        }
+    }
+  };
+  typedef std::integral_constant<int, 0> I0;
+  typedef std::integral_constant<int, W / 2> IH;
+  typedef std::integral_constant<int, W> IW;
+  auto upd_mul = [&](int idx, T (&x)[4][TC]) { upd_mul_part(idx, x, I0(), IW()); };
+  auto upd_store = [&](int idx, T (&x)[4][TC]) {
+    const int rb = idx % RPT, n0 = idx / RPT * W;
+    const unsigned live = upd_live(rb);
+    T *cb = wrows + (int64_t)(64 * rb + rg) * pa.lda + upd.c1 + n0 + cg;
+    if (n0 + W <= upd.rest) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (live >> i & 1u) __builtin_memcpy(cb + i * pa.lda, x[i], sizeof(T) * TC);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int q = 0; q < TC; ++q)
+          if ((live >> i & 1u) && n0 + cg + q < upd.rest) cb[i * pa.lda + q] = x[i][q];
+    }
+  };
+
+  for (int c0 = 0; c0 < pa.npiv && !bail; c0 += W) {
+    const int sub = c0 / W;
+    T *const s_lc = s_l;
+    const int cw = min(W, ncols - c0);    // columns of the sub-panel
+    const int np = min(W, pa.npiv - c0);  // pivots of the sub-panel
+    uint32_t now[RPT];                    // rows that became pivot rows in this sub-panel
+    T v[RPT][W];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int s = 0; s < RPT; ++s) {
+      now[s] = 0u;
+#pragma unroll
+      for (int c = 0; c < W; ++c) v[s][c] = s_l[c * LP + r0 + 64 * s];
+    }
+    // Blocks of the previous sub-panel's update put off into this loop.
+    const int nput = S::kDefer ? upd.next + 1 : 0;
+    T cput[4][TC];
+    if (S::kDefer && nput > 0) upd_fetch(upd.next + RPT, cput);
+
+#pragma unroll 1
+    for (int j = 0; j < np; ++j) {
+      const int par = j & 1, jj = c0 + j, d = pa.row0 + jj;
+      // The wave's candidate: largest |a| > 0, lowest position on ties.
+      {
+        uint32_t kh[RPT], km;
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) {
+          kh[s] = key_hi(v[s][0]) & amask[s];
+          km = s == 0 ? kh[0] : (km > kh[s] ? km : kh[s]);
+        }
+        const uint32_t mh = lanes_max_u32<4>(km);
+        unsigned long long b[RPT];
+        int holders = 0;
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) {
+          b[s] = __builtin_amdgcn_ballot_w64(kh[s] == mh);
+          holders += __popcll(b[s]);
+        }
+        int sw = 0, wl;
+#pragma unroll
+        for (int s = 1; s < RPT; ++s) sw = b[s] ? s : sw;
+        {
+          unsigned long long bb = b[0];
+#pragma unroll
+          for (int s = 1; s < RPT; ++s) bb |= b[s];
+          wl = __ffsll((long long)bb) - 1;
+        }
+        uint32_t *dst = s_c + (par * NWV + wave) * RW;
+        if (__builtin_expect(key_rare<R>(mh, holders), 0)) {
+          R key = R(0);
+          int pos = INT_MAX, sb = 0;
+#pragma unroll
+          for (int s = 0; s < RPT; ++s) {
+            const R k = amask[s] ? rp_key(v[s][0]) : R(0);
+            const bool better = k > key || (k == key && k > R(0) && cpos[s] < pos);
+            key = better ? k : key;
+            pos = better ? cpos[s] : pos;
+            sb = better ? s : sb;
+          }
+          wl = wave_best<R>(key, pos);
+          if (wl < 0) {
+            // No candidate: an entry of zero, which no pick takes.
+            if (lane == 0) {
+              *reinterpret_cast<T *>(dst) = T(0);
+              dst[PW] = (uint32_t)INT_MAX;
+            }
+          } else {
+            sw = __builtin_amdgcn_readlane(sb, wl);
+          }
+        }
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) {
+          if (sw == s && lane == wl) {
+#pragma unroll
+            for (int c = 0; c < W; ++c) reinterpret_cast<T *>(dst)[c] = v[s][c];
+            dst[PW] = (uint32_t)cpos[s];
+            dst[OW] = (uint32_t)(base + r0 + 64 * s);
+          }
+        }
+      }
+      __syncthreads();  // B1
+      // The workgroup's candidate (the same choice among the waves' records).
+      const uint32_t *rec = s_c + par * NWV * RW;
+      int pw;
+      bool none = false;
+      {
+        const uint32_t *rq = rec + min(lane, NWV - 1) * RW;
+        int p = (int)rq[PW];
+        T e0 = *reinterpret_cast<const T *>(rq);
+        pin(p);
+        pin(e0);
+        const uint32_t kh = key_hi(e0) & wmask;
+        const uint32_t mh = lanes_max_u32<1>(kh);
+        const unsigned long long b = __builtin_amdgcn_ballot_w64(kh == mh) & 0xFFFFull;
+        int q = __ffsll((long long)b) - 1;
+        if (__builtin_expect(key_rare<R>(mh, __popcll(b)), 0)) {
+          q = wave_best<R>(wmask && p != INT_MAX ? rp_key(e0) : R(0), p);
+          none = q < 0;
+          q = none ? 0 : q;
+        }
+        pw = __builtin_amdgcn_readlane(p, q);
+        rec += q * RW;
+      }
+      bool due = false;
+      if constexpr (MULTI) {
+        const uint32_t tg = pa.seq + (uint32_t)jj + 1u;
+        unsigned long long *rb = pa.rec + (size_t)par * kMaxPanelWG * kRpRecWords + lane;
+        // Without a candidate every wave's record says so.
+        if (wave == 0) st_agent(rb + g * kRpRecWords, tagged(tg, rec[min(lane, NW)]));
+        // While the records travel: a block of the update put off, if one is
+        // due; the loads go out in its middle, when the other records are
+        // most likely there.
+        due = S::kDefer && upd.next >= 0 && (nput - upd.next) * np <= nput * (j + 1);
+        if constexpr (S::kDefer)
+          if (due) upd_mul_part(upd.next + RPT, cput, I0(), IH());
+        // Every wave takes the records wave, wave + NWV, ...
+        unsigned long long w[MULTI ? MR : 1];
+        auto poll = [&] {
+#pragma unroll
+          for (int i = 0; i < MR; ++i) w[i] = ld_agent(rb + min(wave + i * NWV, pa.P - 1) * kRpRecWords);
+        };
+        poll();
+        if constexpr (S::kDefer)
+          if (due) upd_mul_part(upd.next + RPT, cput, IH(), IW());
+        for (int spins = 0;;) {
+          bool ok = true;
+#pragma unroll
+          for (int i = 0; i < MR; ++i) ok = ok && (uint32_t)(w[i] >> 32) == tg;
+          if (__builtin_expect(__all(ok), 1)) break;
+          ++spins;
+          if (__builtin_expect(spins >= pa.wait_limit || ((spins & 63) == 0 && ld_agent(pa.err) != 0), 0)) {
+            if (lane == 0) {
+              s_bail = 1;
+              atomic_or_agent(pa.err, kErrWait);
+            }
+            break;
+          }
+          poll();
+        }
+        uint32_t *rr = s_r + par * (MR * NWV) * RW;
+#pragma unroll
+        for (int i = 0; i < MR; ++i) rr[(wave + i * NWV) * RW + min(lane, NW)] = (uint32_t)w[i];
+        __syncthreads();  // B2
+        const uint32_t *rq = rr + min(lane, pa.P - 1) * RW;
+        int p = (int)rq[PW], bl = s_bail;
+        T e0 = *reinterpret_cast<const T *>(rq);
+        pin(p);
+        pin(bl);
+        pin(e0);
+        bail = bl != 0;
+        none = false;
+        constexpr int LR = MR * NWV <= 16 ? 1 : 4;
+        const uint32_t kh = key_hi(e0) & pmask;
+        const uint32_t mh = lanes_max_u32<LR>(kh);
+        const unsigned long long b = __builtin_amdgcn_ballot_w64(kh == mh) & (LR == 1 ? 0xFFFFull : ~0ull);
+        int q = __ffsll((long long)b) - 1;
+        if (__builtin_expect(key_rare<R>(mh, __popcll(b)), 0)) {
+          q = wave_best<R>(pmask && p != INT_MAX ? rp_key(e0) : R(0), p);
+          none = q < 0;
+          q = none ? 0 : q;
+        }
+        pw = __builtin_amdgcn_readlane(p, q);
+        rec = rr + q * RW;
+        if (__builtin_expect(bail, 0)) break;
+      }
+      if (__builtin_expect(!none, 1)) {
+        // The multipliers of column j and the update of the columns right of
+        // it (getrf.rs:76-88).  One address register, the whole record in
+        // flight at once.
+        unsigned off = (unsigned)(reinterpret_cast<const unsigned char *>(rec) - smem_raw);
+        __asm__ volatile("" : "+v"(off));
+        const unsigned char *rv = smem_raw + off;
+        T u[W];
+        lds_get<T, W>(u, reinterpret_cast<const T *>(rv));
+        const T ul = reinterpret_cast<const T *>(rv)[min(lane, W - 1)];
+        const int po = (int)reinterpret_cast<const uint32_t *>(rv)[OW];
+        __builtin_amdgcn_sched_barrier(0);
+        const T ur = rp_recip(u[0]);  // (fills the wait for the rest of the record)
+        // U's row j, kept for the sub-panel's store, and the pivot's place.
+        s_u11[j * W + min(lane, W - 1)] = ul;
+        s_po[jj] = po;
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) {
+          const T l = v[s][0] * ur;
+          s_l[j * LP + r0 + 64 * s] = l;
+#pragma unroll
+          for (int c = 1; c < W; ++c) {
+            const T e = l * u[c];
+            v[s][c - 1] = v[s][c] - e;
+          }
+        }
+      } else {
+        // A column without a nonzero candidate is left unscaled
+        // (getrf.rs:72-73); the row at position d is the pivot row.
+        pw = d;
+        last_none = d;
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) {
+          s_l[j * LP + r0 + 64 * s] = v[s][0];
+          if (cpos[s] == d) {
+            s_po[jj] = base + r0 + 64 * s;
+#pragma unroll
+            for (int c = 0; c < W; ++c) s_u11[j * W + c] = v[s][c];
+          }
+#pragma unroll
+          for (int c = 1; c < W; ++c) v[s][c - 1] = v[s][c];
+        }
+      }
+      if constexpr (S::kDefer) {
+        if (due) {
+          upd_store(upd.next + RPT, cput);
+          --upd.next;
+          upd_fetch(max(upd.next, 0) + RPT, cput);
+        }
+      }
+      s_pw[jj] = pw;
+      // Interchange bookkeeping: the pivot row takes position d, the row at d
+      // takes the pivot's old position (rows retired earlier lie above d).
+#pragma unroll
+      for (int s = 0; s < RPT; ++s) {
+        const bool hit = cpos[s] == pw;
+        now[s] = hit ? 1u : now[s];
+        amask[s] = hit ? 0u : amask[s];
+        cpos[s] = cpos[s] == d ? pw : cpos[s];
+        cpos[s] = hit ? d : cpos[s];
+      }
+      done = jj + 1;
+    }
+    if (bail) break;
+
+    // Opaque copies of the lane and the row pitch keep the addresses and masks
+    // of the phases between the column loops from being computed ahead of the
+    // loops and held in registers through them.
+    if constexpr (S::kDefer) {
+      for (; upd.next >= 0; --upd.next) {
+        upd_mul(upd.next + RPT, cput);
+        upd_store(upd.next + RPT, cput);
+        upd_fetch(max(upd.next - 1, 0) + RPT, cput);
+      }
+    }
+    int lane_o = lane;
+    int64_t lda_o = pa.lda;
+    __asm__ volatile("" : "+v"(lane_o));
+    __asm__ volatile("" : "+s"(lda_o));
+    unsigned long long m_live[RPT], m_store[RPT];
+#pragma unroll
+    for (int s = 0; s < RPT; ++s) {
+      m_live[s] = __builtin_amdgcn_ballot_w64(amask[s] != 0u);
+      m_store[s] = m_live[s] | __builtin_amdgcn_ballot_w64(now[s] != 0u);
+    }
+    const int c1 = c0 + W, rest = ncols - c1;
+    const int un = (rest + 3) & ~3;  // pitch of U in LDS
+    __syncthreads();
+    // U11's rows into the tile, at the rows that own them.
+    if (t < np * W) {
+      const int j = t / W, c = t % W, pt = s_po[c0 + j] - base;
+      if ((unsigned)pt < (unsigned)NR) {
+        if (c >= j) s_l[c * LP + pt] = s_u11[j * W + c - j];
+        // L11, when all of it is this workgroup's.
+        if (!MULTI && rest > 0 && c < j) s_lt[j * W + c] = s_l[c * LP + pt];
+      }
+    }
+    if (rest > 0) {
+      // The pivot rows' multipliers and their entries right of the sub-panel.
+      if constexpr (!MULTI) {
+        raw_t x[JW][2];
+#pragma unroll
+        for (int i = 0; i < JW; ++i) {
+          const int j = min(wave + i * NWV, np - 1);
+          const T *src = rows + (int64_t)(s_po[c0 + j] - base) * lda_o + c1;
+#pragma unroll
+          for (int e = 0; e < 2; ++e) x[i][e] = *reinterpret_cast<const raw_t *>(src + min(lane_o + 64 * e, rest - 1));
+        }
+#pragma unroll
+        for (int i = 0; i < JW; ++i) {
+          const int j = min(wave + i * NWV, np - 1);
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            *reinterpret_cast<raw_t *>(s_u + j * un + min(lane_o + 64 * e, rest - 1)) = x[i][e];
+        }
+      } else {
+        const uint32_t tb = pa.seq + kRpTagBlk + (uint32_t)sub;
+        unsigned long long *bb = pa.blk + (size_t)(sub & 1) * kRpMaxW * kRpRowWords;
+        const int rw = EW + rest * WPE;  // words per pivot row
+        for (int j = wave; j < np; j += NWV) {
+          const int pt = s_po[c0 + j] - base;
+          if ((unsigned)pt >= (unsigned)NR) continue;
+          const uint32_t *src = reinterpret_cast<const uint32_t *>(rows + (int64_t)pt * lda_o + c1) - EW;
+          uint32_t x[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int k = min(lane_o + 64 * e, rw - 1);
+            x[e] = src[max(k, EW)];
+            const uint32_t y = reinterpret_cast<const uint32_t *>(s_l + (min(k, EW - 1) / WPE) * LP + pt)[k % WPE];
+            x[e] = k < EW ? y : x[e];
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int k = min(lane_o + 64 * e, rw - 1);
+            st_agent(bb + (size_t)j * kRpRowWords + k, tagged(tb, x[e]));
+          }
+        }
+        unsigned long long w[JW][4];
+        int spins = 0;
+        for (;;) {
+          bool ok = true;
+#pragma unroll
+          for (int i = 0; i < JW; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              w[i][e] = ld_agent(bb + (size_t)min(wave + i * NWV, np - 1) * kRpRowWords + min(lane_o + 64 * e, rw - 1));
+#pragma unroll
+          for (int i = 0; i < JW; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ok = ok && (uint32_t)(w[i][e] >> 32) == tb;
+          if (__all(ok)) break;
+          ++spins;
+          if (spins >= pa.wait_limit || ((spins & 63) == 0 && ld_agent(pa.err) != 0)) {
+            if (lane_o == 0) {
+              s_bail = 1;
+              atomic_or_agent(pa.err, kErrWait);
+            }
+            break;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < JW; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int j = min(wave + i * NWV, np - 1), k = min(lane_o + 64 * e, rw - 1);
+            *(k < EW ? reinterpret_cast<uint32_t *>(s_lt + j * W) + k
+                     : reinterpret_cast<uint32_t *>(s_u + j * un) + (k - EW)) = (uint32_t)w[i][e];
+          }
+      }
+    }
+    __syncthreads();
+    bail = s_bail != 0;
+    if (bail) break;
+    // The sub-panel back to the matrix (rows retired earlier already hold
+    // their final entries there).
+    {
+      const int wc = lane_o % W, wr = lane_o / W;
+#pragma unroll
+      for (int s = 0; s < RPT; ++s) {
+        const unsigned long long ms = wc < cw ? m_store[s] >> wr : 0ull;
+        T *dst = wrows + (int64_t)(64 * s + wr) * lda_o + c0 + wc;
+        T x[W];
+#pragma unroll
+        for (int i = 0; i < W; ++i) x[i] = s_l[wc * LP + wave * WR + 64 * s + wr + i * RS];
+#pragma unroll
+        for (int i = 0; i < W; ++i)
+          if (ms >> (i * RS) & 1ull) dst[i * RS * lda_o] = x[i];
+      }
+    }
+    if (rest <= 0) break;
+    // U = L11^-1 A, one thread per column.
+    if (t < rest) {
+      T x[W];
+#pragma unroll
+      for (int i = 0; i < W; ++i) x[i] = s_u[i * un + t];
+#pragma unroll
+      for (int i = 1; i < W; ++i) {
+        T l[W];
+#pragma unroll
+        for (int q = 0; q < i; ++q) l[q] = s_lt[i * W + q];
+#pragma unroll
+        for (int q = 0; q < i; ++q) {
+          const T e = l[q] * x[q];
+          x[i] = x[i] - e;
+        }
+        // Two rows of L11 at a time in registers.
+        if (i % 2 == 0) __asm__ volatile("" : "+v"(reinterpret_cast<uint32_t &>(x[i])) : : "memory");
+      }
+#pragma unroll
+      for (int i = 1; i < W; ++i)
+        if (i < np) s_u[i * un + t] = x[i];
+    }
+    __syncthreads();
+    // The pivot rows' entries right of the sub-panel, by their owners.
+#pragma unroll
+    for (int i = 0; i < JW; ++i) {
+      const int j = wave + i * NWV, pt = j < np ? s_po[c0 + j] - base : -1;
+      if ((unsigned)pt < (unsigned)NR) {
+        T *dst = rows + (int64_t)pt * lda_o + c1;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          if (lane_o + 64 * e < rest) dst[lane_o + 64 * e] = s_u[j * un + lane_o + 64 * e];
+      }
+    }
+    // A22 -= L21 U on this wave's rows.  The next sub-panel's columns come
+    // last and stay in LDS; with kDefer the whole blocks beyond them wait.
+    upd.c1 = c1;
+    upd.rest = rest;
+    upd.un = un;
+    upd.l = s_lc;
+#pragma unroll
+    for (int s = 0; s < RPT; ++s) upd.live[s] = m_live[s];
+    if constexpr (S::kDefer) {
+      // This tile's L is still needed: the next sub-panel goes to the other.
+      s_l = s_lold;
+      s_lold = s_lc;
+    }
+    {
+      const int whole = rest / W;  // whole blocks of columns
+      T c[4][TC], cnext[4][TC];
+      if (whole * W < rest) {
+        // A ragged last block.
+        for (int rb = RPT - 1; rb >= 0; --rb) {
+          const int idx = whole * RPT + rb;
+          upd_fetch_edge(idx, c);
+          upd_mul(idx, c);
+          if (whole > 0) {
+            upd_store(idx, c);
+          } else {
+            T *dst = s_l + wave * WR + 64 * rb + rg;
+#pragma unroll
+            for (int q = 0; q < TC; ++q)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) dst[(cg + q) * LP + i] = c[i][q];
+          }
+        }
+      }
+      if (whole > 0) {
+        const int last = S::kDefer ? RPT - 1 : whole * RPT - 1;
+        upd_fetch(last, c);
+#pragma unroll 1
+        for (int idx = last; idx >= 0; --idx) {
+          upd_fetch(max(idx - 1, 0), cnext);
+          upd_mul(idx, c);
+          if (idx >= RPT) {
+            upd_store(idx, c);
+          } else {
+            T *dst = s_l + wave * WR + 64 * idx + rg;
+#pragma unroll
+            for (int q = 0; q < TC; ++q)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) dst[(cg + q) * LP + i] = c[i][q];
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int q = 0; q < TC; ++q) c[i][q] = cnext[i][q];
+        }
+      }
+      // The blocks put off: RPT + next, ..., RPT.
+      upd.next = S::kDefer ? max(whole - 1, 0) * RPT - 1 : -1;
+    }
+  }
+  __syncthreads();
+  if (g == 0) {
+    // The pivots.  Given up: identity pivots for the columns not decided keep
+    // the interchanges queued after this launch in bounds.
+    for (int e = t; e < pa.npiv; e += NT) pa.ipiv[pa.row0 + e] = e < done ? s_pw[e] : pa.row0 + e;
+    if (t == 0) {
+      if (last_none >= 0) *pa.sing = last_none;
+      if (pa.map_count) *pa.map_count = bail ? 0 : 2 * pa.npiv;
+    }
+  }
+  if (bail) return;
 
   // Row map of the leaf's interchanges in gather form (rows[e] receives the
   // old contents of src[e]; rows[e] == src[e] is a no-op).  Slot e < npiv:
   // the final occupant of position row0 + e.  Slot npiv + e: where the row
   // that started at row0 + e went, when it left [row0, row0 + npiv).  Each
   // slot is written once, by the owner of the row it describes.
-  if (wave > 0) {
+  const int top1 = pa.row0 + pa.npiv;
+  int *s_mvt = reinterpret_cast<int *>(smem_raw), *s_out = s_mvt + S::MOVED, *s_in = s_out + S::MOVED;
 #pragma unroll
-    for (int s = 0; s < RPT; ++s) {
-      const int orig = base + tw + s * NW;
-      const bool valid = orig < pa.m;
-      s_fin[tw + s * NW] = valid ? cpos[s] : -1;
-      if (pa.map_rows && valid) {
-        const int top1 = pa.row0 + pa.npiv;
-        const int fin = cpos[s];
-        if (fin < top1) {
-          pa.map_rows[fin - pa.row0] = fin;
-          pa.map_src[fin - pa.row0] = orig;
+  for (int s = 0; s < RPT; ++s) {
+    if (r0 + 64 * s >= nvalid) continue;
+    const int orig = base + r0 + 64 * s, fin = cpos[s];
+    if (pa.map_rows) {
+      if (fin < top1) {
+        pa.map_rows[fin - pa.row0] = fin;
+        pa.map_src[fin - pa.row0] = orig;
+      }
+      if (orig < top1) {
+        pa.map_rows[pa.npiv + orig - pa.row0] = fin < top1 ? orig : fin;
+        pa.map_src[pa.npiv + orig - pa.row0] = orig;
+      }
+    }
+    if (fin != orig) {
+      const int k = atomicAdd(&s_cnt, 1);
+      s_mvt[k] = r0 + 64 * s;
+      if constexpr (MULTI) {
+        // This row leaves and another takes its place: the source of a
+        // position is found by walking it back through the interchanges.  A
+        // row's slot: its origin if that is one of the first npiv rows, else
+        // its destination (which then is).
+        int x = orig;
+        for (int e = (pa.npiv - 1) & ~7; e >= 0; e -= 8) {
+          int pe[8];
+          lds_get<int, 8>(pe, s_pw + e);
+#pragma unroll
+          for (int q = 7; q >= 0; --q) {
+            const int de = pa.row0 + e + q, pq = e + q < pa.npiv ? pe[q] : de;
+            x = x == de ? pq : (x == pq ? de : x);
+          }
         }
-        if (orig < top1) {
-          pa.map_rows[pa.npiv + orig - pa.row0] = fin < top1 ? orig : fin;
-          pa.map_src[pa.npiv + orig - pa.row0] = orig;
-        }
+        s_out[k] = orig < top1 ? kRpMaxCols + orig - pa.row0 : fin - pa.row0;
+        s_in[k] = x < top1 ? kRpMaxCols + x - pa.row0 : orig - pa.row0;
+      } else {
+        s_out[k] = fin - base;
       }
     }
   }
-  if (pa.map_count && g == 0 && t == 0) *pa.map_count = 2 * pa.npiv;
   __syncthreads();
-
-  // Write-back: every row to its final position.
-  for (int i = wave; i < R; i += NWK + 1) {
-    const int dst = s_fin[i];
-    if (dst < 0) continue;
-    T *out = pa.a + (int64_t)dst * pa.lda + pa.col0;
+  const int cnt = s_cnt;
+  if (cnt == 0) return;
+  if constexpr (!MULTI) {
+    // Rows within the workgroup: 64 columns at a time through registers, all
+    // loaded before any is stored.  Lanes and rows past the end repeat the
+    // last one.
+    constexpr int BR = 16, NB = (S::MOVED / NWV + BR - 1) / BR;
+    for (int cb = 0; cb < ncols; cb += 64) {
+      const T *src = rows + min(cb + lane, ncols - 1);
+      T *dst = rows + min(cb + lane, ncols - 1);
+      raw_t x[NB][BR];
 #pragma unroll
-    for (int q = 0; q < NI; ++q) {
-      const int c = lane + 64 * q;
-      if (c < ncols) out[c] = s_a[c * LDC + i];
+      for (int b = 0; b < NB; ++b)
+        if (b * BR * NWV < cnt) {
+#pragma unroll
+          for (int i = 0; i < BR; ++i)
+            x[b][i] = *reinterpret_cast<const raw_t *>(
+                src + (int64_t)s_mvt[min(wave + (b * BR + i) * NWV, cnt - 1)] * pa.lda);
+        }
+      // Every load has arrived before the first store.
+      __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        if (b * BR * NWV < cnt) {
+#pragma unroll
+          for (int i = 0; i < BR; ++i)
+            *reinterpret_cast<raw_t *>(dst + (int64_t)s_out[min(wave + (b * BR + i) * NWV, cnt - 1)] * pa.lda) =
+                x[b][i];
+        }
     }
+  } else {
+    // Through the tagged slots, 64 words of 16 rows at a time.
+    constexpr int BR = 16;
+    const int wpr = ncols * WPE;
+    const uint32_t tm = pa.seq + kRpTagMv;
+    for (int e0 = wave; e0 < cnt; e0 += BR * NWV)
+      for (int k0 = 0; k0 < wpr; k0 += 64) {
+        const int k = min(k0 + lane, wpr - 1);
+        uint32_t x[BR];
+#pragma unroll
+        for (int i = 0; i < BR; ++i)
+          x[i] = reinterpret_cast<const uint32_t *>(rows + (int64_t)s_mvt[min(e0 + i * NWV, cnt - 1)] * pa.lda)[k];
+#pragma unroll
+        for (int i = 0; i < BR; ++i)
+          st_agent(pa.mv + (size_t)s_out[min(e0 + i * NWV, cnt - 1)] * kRpRowWords + k, tagged(tm, x[i]));
+      }
+    __syncthreads();
+    for (int e0 = wave; e0 < cnt; e0 += BR * NWV)
+      for (int k0 = 0; k0 < wpr; k0 += 64) {
+        const int k = min(k0 + lane, wpr - 1);
+        unsigned long long w[BR];
+        int spins = 0;
+        for (;;) {
+          bool ok = true;
+#pragma unroll
+          for (int i = 0; i < BR; ++i)
+            w[i] = ld_agent(pa.mv + (size_t)s_in[min(e0 + i * NWV, cnt - 1)] * kRpRowWords + k);
+#pragma unroll
+          for (int i = 0; i < BR; ++i) ok = ok && (uint32_t)(w[i] >> 32) == tm;
+          if (__all(ok)) break;
+          ++spins;
+          if (spins >= pa.wait_limit || ((spins & 63) == 0 && ld_agent(pa.err) != 0)) {
+            if (lane == 0) atomic_or_agent(pa.err, kErrWait);
+            break;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < BR; ++i)
+          reinterpret_cast<uint32_t *>(rows + (int64_t)s_mvt[min(e0 + i * NWV, cnt - 1)] * pa.lda)[k] = (uint32_t)w[i];
+      }
   }
 }
 
-template <typename T, int NB, int NWK, int RPT>
+template <typename T, int RPT, int MR>
 static hipError_t rp_launch(lair_context *ctx, const RpArgs<T> &pa) {
-  auto *k = &rpanel_kernel<T, NB, NWK, RPT>;
-  constexpr int R = 64 * NWK * RPT;
-  const size_t shm = (size_t)NB * (R + 1) * sizeof(T);
+  auto *k = &rpanel_kernel<T, RPT, MR>;
+  constexpr size_t shm = RpLds<T, RPT, MR>::total;
   static bool once = ((void)hipFuncSetAttribute(reinterpret_cast<const void *>(k),
                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                                 (int)shm),
                       (void)hipGetLastError(), true);
   (void)once;
-  k<<<pa.P, 64 * (NWK + 1), shm, ctx->stream>>>(pa);
+  k<<<pa.P, kRpThreads, shm, ctx->stream>>>(pa);
   return hipGetLastError();
 }
 
+// Rows per thread of a leaf over `rows` rows, or 0 when the leaf does not fit
+// the cooperating workgroups.
 template <typename T>
-int rpanel_rows_per_wg(lair_context *ctx, int nbw, int rows) {
+static int rp_rpt(lair_context *ctx, int rows) {
   const int maxp = std::min(ctx->rp_max_wg, kMaxPanelWG);
-  // {leaf width, rows per workgroup}: the rows of a workgroup fill about
-  // 130 KB of LDS, and a header or row record fits its exchange slot.
-  static const int kF[][2] = {{128, 256}, {64, 512}, {32, 1024}};
-  static const int kD[][2] = {{64, 256}, {32, 512}, {16, 1024}};
-  static const int kC[][2] = {{64, 256}, {32, 512}, {16, 1024}};  // complex<float>
-  static const int kZ[][2] = {{32, 256}, {16, 512}, {0, 0}};      // complex<double>
-  const auto &tab = sizeof(T) == 4 ? kF : sizeof(T) == 16 ? kZ : cplx_traits<T>::is ? kC : kD;
-  for (const auto &e : tab)
-    if (e[0] > 0 && e[0] == nbw && (rows + e[1] - 1) / e[1] <= maxp) return e[1];
-  return 0;
+  // Complex<f64> keeps to 32768 rows, the limit its entry points state.
+  if (sizeof(T) == 16 && rows > 32768) return 0;
+  if (rows <= kRpThreads) return 1;
+  if (rows <= 2 * kRpThreads) return 2;
+  if (rows <= 4 * kRpThreads) return 4;
+  if (rows <= 2 * kRpThreads * std::min(maxp, 32)) return 2;
+  return rows <= 4 * kRpThreads * maxp ? 4 : 0;
 }
 
-// Widest leaf (<= want) that the resident kernel can factor for `rows` rows.
+template <typename T>
+int rpanel_grid(lair_context *ctx, int rows) {
+  const int nr = rp_rpt<T>(ctx, rows) * kRpThreads;
+  return nr > 0 ? (rows + nr - 1) / nr : 0;
+}
+
+// Widest leaf (<= want) for `rows` rows.
 template <typename T>
 int rpanel_leaf_width(lair_context *ctx, int want, int rows) {
-  for (int w : {128, 64, 32, 16})
-    if (w <= want && rpanel_rows_per_wg<T>(ctx, w, rows) > 0) return w;
-  return 0;
+  return rpanel_grid<T>(ctx, rows) > 0 ? std::min(want, RpLds<T, 1, 0>::NBM) : 0;
 }
 
 template <typename T>
 hipError_t launch_rpanel(lair_context *ctx, T *a, int64_t lda, int row0, int m, int col0, int wcols,
-                         int nbw, int64_t *ipiv, int *map_rows, int *map_src, int *map_count) {
+                         int64_t *ipiv, int *map_rows, int *map_src, int *map_count) {
   const int rows = m - row0;
   if (rows <= 0 || wcols <= 0) return hipSuccess;
-  if (wcols > nbw || m >= (int)kRpNone) return hipErrorInvalidValue;
-  const int R = rpanel_rows_per_wg<T>(ctx, nbw, rows);
-  if (R == 0) return hipErrorInvalidValue;
-  // Header tags carry 16 bits: start a new tag epoch (cleared slots) before
-  // they could wrap inside this launch.
-  if ((ctx->rp_seq & 0xFFFFu) + (uint32_t)nbw + 2u > 0xFFFFu || ctx->rp_seq > 0xF0000000u) {
-    hipError_t e = launch_fill_u32(ctx, reinterpret_cast<uint32_t *>(ctx->rp_hdr),
-                                   2 * kRpHdrTotal, 0u);
-    if (e == hipSuccess)
-      e = launch_fill_u32(ctx, reinterpret_cast<uint32_t *>(ctx->rp_rowd),
-                          2 * 2 * kMaxPanelWG * kRpRowWords, 0u);
+  const int rpt = rp_rpt<T>(ctx, rows);
+  if (rpt == 0 || wcols > RpLds<T, 1, 0>::NBM) return hipErrorInvalidValue;
+  // A reused tag could match a stale word: clear the buffers and restart the
+  // tags before they wrap.
+  if (ctx->rp_seq > 0xF0000000u) {
+    hipError_t e = launch_fill_u32(ctx, reinterpret_cast<uint32_t *>(ctx->rp_buf), 2 * kRpBufWords, 0u);
     if (e != hipSuccess) return e;
-    ctx->rp_seq = ctx->rp_seq > 0xF0000000u ? 1u : ((ctx->rp_seq | 0xFFFFu) + 2u);
+    ctx->rp_seq = 1u;
   }
   RpArgs<T> pa;
   pa.a = a;
@@ -651,62 +1043,41 @@ hipError_t launch_rpanel(lair_context *ctx, T *a, int64_t lda, int row0, int m, 
   pa.col0 = col0;
   pa.wcols = wcols;
   pa.npiv = wcols < rows ? wcols : rows;
-  pa.P = (rows + R - 1) / R;
+  pa.P = rpanel_grid<T>(ctx, rows);
   pa.ipiv = ipiv;
   pa.sing = ctx->sing;
   pa.map_rows = map_rows;
   pa.map_src = map_src;
   pa.map_count = map_count;
-  pa.hdr = ctx->rp_hdr + (cplx_traits<T>::is ? kRpHdrComplexOff : 0);
-  pa.rowd = ctx->rp_rowd;
+  pa.rec = ctx->rp_buf;
+  pa.blk = ctx->rp_buf + kRpBlkOff;
+  pa.mv = ctx->rp_buf + kRpMvOff;
   pa.seq = ctx->rp_seq;
   pa.err = ctx->err;
   pa.wait_limit = ctx->wait_limit;
   const int slot = prof_begin(ctx, LAIR_KCLASS_PANEL);
   hipError_t e;
-  if constexpr (sizeof(T) == 16) {
-    if (nbw == 32) e = rp_launch<T, 32, 4, 1>(ctx, pa);
-    else e = rp_launch<T, 16, 4, 2>(ctx, pa);
-  } else if constexpr (cplx_traits<T>::is) {
-    if (nbw == 64) e = rp_launch<T, 64, 4, 1>(ctx, pa);
-    else if (nbw == 32) e = rp_launch<T, 32, 4, 2>(ctx, pa);
-    else e = rp_launch<T, 16, 4, 4>(ctx, pa);
-  } else if constexpr (sizeof(T) == 4) {
-    if (nbw == 128) e = rp_launch<T, 128, 4, 1>(ctx, pa);
-    else if (nbw == 64) e = rp_launch<T, 64, 4, 2>(ctx, pa);
-    else e = rp_launch<T, 32, 4, 4>(ctx, pa);
-  } else {
-    if (nbw == 64) e = rp_launch<T, 64, 4, 1>(ctx, pa);
-    else if (nbw == 32) e = rp_launch<T, 32, 4, 2>(ctx, pa);
-    else e = rp_launch<T, 16, 4, 4>(ctx, pa);
-  }
+  if (pa.P == 1)
+    e = rpt == 1 ? rp_launch<T, 1, 0>(ctx, pa) : (rpt == 2 ? rp_launch<T, 2, 0>(ctx, pa) : rp_launch<T, 4, 0>(ctx, pa));
+  else if (rpt == 4)
+    e = rp_launch<T, 4, 16>(ctx, pa);
+  else if (pa.P <= 8)
+    e = pa.P <= 4 ? rp_launch<T, 2, 1>(ctx, pa) : rp_launch<T, 2, 2>(ctx, pa);
+  else
+    e = pa.P <= 16 ? rp_launch<T, 2, 4>(ctx, pa) : rp_launch<T, 2, 8>(ctx, pa);
   prof_end(ctx, slot, LAIR_KCLASS_PANEL, (double)pa.npiv * rows * wcols,
            2.0 * sizeof(T) * (double)rows * wcols);
-  ctx->rp_seq += (uint32_t)nbw + 1u;
+  ctx->rp_seq += kRpTags;
   return e;
 }
 
-template <typename T>
-int rpanel_grid(lair_context *ctx, int nbw, int rows) {
-  const int R = rpanel_rows_per_wg<T>(ctx, nbw, rows);
-  return R > 0 ? (rows + R - 1) / R : 0;
-}
-
-template int rpanel_grid<float>(lair_context *, int, int);
-template int rpanel_grid<double>(lair_context *, int, int);
-template int rpanel_leaf_width<float>(lair_context *, int, int);
-template int rpanel_leaf_width<double>(lair_context *, int, int);
-template hipError_t launch_rpanel<float>(lair_context *, float *, int64_t, int, int, int, int, int,
-                                         int64_t *, int *, int *, int *);
-template hipError_t launch_rpanel<double>(lair_context *, double *, int64_t, int, int, int, int, int,
-                                          int64_t *, int *, int *, int *);
-template int rpanel_grid<zcplx>(lair_context *, int, int);
-template int rpanel_grid<ccplx>(lair_context *, int, int);
-template int rpanel_leaf_width<zcplx>(lair_context *, int, int);
-template int rpanel_leaf_width<ccplx>(lair_context *, int, int);
-template hipError_t launch_rpanel<zcplx>(lair_context *, zcplx *, int64_t, int, int, int, int, int, int64_t *,
-                                         int *, int *, int *);
-template hipError_t launch_rpanel<ccplx>(lair_context *, ccplx *, int64_t, int, int, int, int, int, int64_t *,
-                                         int *, int *, int *);
+#define LAIR_RP_INST(T)                                                                                \
+  template int rpanel_grid<T>(lair_context *, int);                                                    \
+  template int rpanel_leaf_width<T>(lair_context *, int, int);                                         \
+  template hipError_t launch_rpanel<T>(lair_context *, T *, int64_t, int, int, int, int, int64_t *, int *, int *, int *);
+LAIR_RP_INST(float)
+LAIR_RP_INST(double)
+LAIR_RP_INST(zcplx)
+LAIR_RP_INST(ccplx)
 
 }  // namespace lair

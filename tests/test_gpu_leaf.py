@@ -1,0 +1,76 @@
+"""The panel leaf (rpanel.hip) at the sizes where its plan changes: one
+workgroup with 1, 2 or 4 rows per thread (256, 512, 1024 rows), several
+workgroups (from 1025 rows, by the number of records a wave polls: 2048, 4096,
+8192 rows; from 16385 with 4 rows per thread), sub-panels of 16 (complex<f64>:
+8) columns and ragged last ones.
+
+A matrix of at most 64 columns is one leaf, whose operations are those of
+getrf_row_major (src/lapack/getrf.rs:55-117) in the same order, so pivots and
+factors have to equal the oracle's bit for bit; no tolerance is involved.
+"""
+import numpy as np
+import pytest
+
+import lair_amd as L
+from lair_amd import inputs
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1), (15, 16), (16, 15), (17, 33), (255, 64), (256, 16), (257, 17), (512, 64), (513, 31), (1023, 48),
+          (1024, 64), (1025, 64), (2048, 16), (2049, 33), (4097, 40), (8193, 24), (16385, 20), (64, 300)]
+ORACLE = {np.float64: O.getrf, np.float32: O.sgetrf, np.complex128: O.zgetrf, np.complex64: O.cgetrf}
+TYPES = list(ORACLE)
+
+
+def _same_as_oracle(a, cols):
+    ref = a.copy()
+    piv_o, sing_o = ORACLE[a.dtype.type](ref)
+    g = a.copy()
+    piv, sing = L.getrf(g)
+    assert np.array_equal(piv, piv_o)
+    assert sing == sing_o
+    assert np.array_equal(g[:, :cols], ref[:, :cols], equal_nan=True)
+
+
+def _gauss(seed, m, n, dt):
+    a = inputs.gaussian_matrix(seed, m, n)
+    if np.dtype(dt).kind == "c":
+        a = a + 1j * inputs.gaussian_matrix(seed + 1, m, n)
+    return a.astype(dt)
+
+
+@pytest.mark.parametrize("dt", TYPES)
+@pytest.mark.parametrize("shape", SHAPES)
+def test_leaf_equals_oracle(shape, dt):
+    m, n = shape
+    _same_as_oracle(_gauss(500 + m + n, m, n, dt), min(n, 64))
+
+
+@pytest.mark.parametrize("dt", TYPES)
+@pytest.mark.parametrize("m", [300, 700, 1500])
+def test_leaf_ties_and_empty_columns(m, dt):
+    """Small integers (most columns hold equal maxima, in one wave, across
+    waves and across workgroups) and columns without a candidate, first and
+    last in a sub-panel."""
+    rng = np.random.default_rng(m)
+    a = rng.integers(-2, 3, (m, 40)).astype(np.float64)
+    if np.dtype(dt).kind == "c":
+        a = a + 1j * rng.integers(-2, 3, (m, 40))
+    a = a.astype(dt)
+    for c in (0, 7, 15, 16, 31):
+        a[:, c] = 0
+    _same_as_oracle(a, 40)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("m", [200, 1300])
+def test_leaf_extreme_values(m, dt):
+    """Infinities, NaN (never chosen) and subnormal entries among the candidates."""
+    tiny = np.finfo(dt).smallest_subnormal
+    a = _gauss(900 + m, m, 20, dt)
+    a[:, 0] = 0
+    a[m - 3, 0], a[5, 0], a[m // 2, 0] = 3 * tiny, 2 * tiny, -3 * tiny
+    a[7, 4] = np.nan
+    a[m - 1, 9] = np.inf
+    _same_as_oracle(a, 20)
