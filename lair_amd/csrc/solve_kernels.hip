@@ -941,9 +941,9 @@ __device__ __forceinline__ void trsv_block(const TrsvArgs<T> &p, int wid, const 
   }
 }
 
-template <typename T, int BS, int RC>
+template <typename T, int BS>
 __global__ void __launch_bounds__(256) trsv_dataflow_kernel(TrsvArgs<T> p) {
-  trsv_block<T, BS, RC, false>(p, blockIdx.x, IrFuse{});
+  trsv_block<T, BS, 1, false>(p, blockIdx.x, IrFuse{});
 }
 
 // Residual workgroup rw of the fused refinement step: rows
@@ -1165,26 +1165,59 @@ __global__ void __launch_bounds__(256) trsv_ir_kernel(TrsvArgs<float> p, IrFuse 
     ir_residual_block<RC>(p, f, blockIdx.x - ntri);
 }
 
-// Many right-hand sides in FP32 (nrhs >= 16, not transposed): the same
-// dataflow as trsv_dataflow_kernel (one workgroup per 128-row block and
-// 16-column chunk, solved values published as tagged words), with the block
-// products on matrix cores.  Wave w owns rows 32w .. 32w + 31 of the block
-// as two 16 x 16 v_mfma_f32_16x16x4f32 accumulators, so a workgroup needs
-// few registers and two fit on a CU (all 512 workgroups of a 64-column solve
-// at n = 16384 are resident at once).
-//  * E_ij tiles (128 x 128) are staged through registers into LDS, 16-byte
-//    chunk c of row r at chunk position c ^ (r & 31); MFMA step s takes
-//    k = 16 t + 4 g + s from lane group g, so a lane's four k values are one
-//    16-byte LDS read and the 16 rows read together are on distinct banks.
-//  * -X_j is staged transposed ([column][k]), so acc = b - sum E_ij X_j.
-//  * D_i^-1 (the inverted diagonal block) stays in registers in the MFMA
-//    operand layout; y goes through LDS as the second operand of x = D y.
-__global__ void __launch_bounds__(256, 2) trsm_mfma_kernel(TrsvArgs<float> p) {
-  constexpr int BS = 128, RC = 16, XP = BS + 4;
-  typedef float f4 __attribute__((ext_vector_type(4)));
+// Matrix-core dataflow solve for several right-hand sides: workgroup (block
+// row i, chunk of 16 columns) keeps its BS x 16 right-hand sides in MFMA
+// accumulators (a wave BS / 4 rows by 16 columns), subtracts E_ij X_j for the
+// blocks j solved before it and applies the inverted diagonal block.
+//  * E_ij tiles are staged through registers into LDS as they lie in memory
+//    (pitch BS + 16 bytes: the 16 rows, or with TRANS columns, that an MFMA
+//    operand reads together are on distinct banks).  MFMA step (s, ks) takes
+//    k = 16 s + 4 g + ks from lane group g.
+//  * -X_j is staged transposed ([column][k]), so acc = b - sum E_ij X_j.  Its
+//    tagged words are all requested at once, eight per thread (bounded
+//    polls): one round trip per block, not one per word.
+//  * Every block's product is four (FP32: two) partial sums added pairwise
+//    before they meet the right-hand side, so rounding grows with the number of
+//    blocks and not with n (one running accumulator: 1.35 times the error).
+//  * D_i^-1 stays in registers in the MFMA operand layout; y goes through LDS
+//    as the second operand of x = D y.
+// Bound by the chain of blocks: one round trip of the words (0.8 us), the
+// products with the last block and with D (0.4 us each in FP64) and their
+// barriers: 3.2 us per block in FP64.  Both solves of n = 4096 with 64
+// right-hand sides: 0.50 ms, where the vector kernel took 1.88 ms (14.7 us
+// per block); with 16: 0.42 ms against 1.03.
+template <typename T>
+struct TrsmMfma;
+template <>
+struct TrsmMfma<double> {
+  typedef double v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ v4 op(double a, double b, v4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int g, int r) { return g + 4 * r; }
+};
+template <>
+struct TrsmMfma<float> {
+  typedef float v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ v4 op(float a, float b, v4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int g, int r) { return 4 * g + r; }
+};
+
+template <typename T, int BS, bool TRANS>
+__global__ void __launch_bounds__(256, 2) trsm_mfma_kernel(TrsvArgs<T> p) {
+  typedef TrsmMfma<T> M;
+  typedef typename M::v4 v4;
+  constexpr int RC = 16, WPE = sizeof(T) / 4, VEC = 16 / sizeof(T), P = BS + VEC;
+  constexpr int RB = BS / 64, KS = BS / 16;        // row blocks of a wave, k groups of 16
+  constexpr int NC = 256 / BS;                     // partial sums of a product
+  constexpr int NV = BS * BS / VEC / 256;          // 16-byte loads per thread per tile
+  constexpr int NWD = BS * RC * WPE / 256;         // tagged words per thread per block
+  typedef T vec_t __attribute__((ext_vector_type(VEC)));
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  float *tile = reinterpret_cast<float *>(smem_raw);  // [BS][BS], swizzled 16-byte chunks
-  __shared__ __align__(16) float xs[RC][XP];          // B operand, transposed
+  T *tile = reinterpret_cast<T *>(smem_raw);       // [BS][P], as in memory
+  __shared__ __align__(16) T xs[RC][P];            // second operand, transposed
   __shared__ int s_bail;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int g = lane >> 4, lc = lane & 15;
@@ -1192,49 +1225,70 @@ __global__ void __launch_bounds__(256, 2) trsm_mfma_kernel(TrsvArgs<float> p) {
   const int i = p.forward ? ib : p.nblk - 1 - ib;
   const int r0 = i * BS, c0 = ch * RC;
   const int ncols = p.nrhs - c0 < RC ? p.nrhs - c0 : RC;
-  auto swz = [](int r, int c4) { return r * BS + ((c4 ^ (r & 31)) << 2); };
-  // Rows of this lane's accumulator element (rb, r).
-  auto arow = [&](int rb, int r) { return 32 * wave + 16 * rb + 4 * g + r; };
+  const int wrow = wave * (BS / 4);                // this wave's first row
+  auto arow = [&](int rb, int r) { return wrow + 16 * rb + M::row(g, r); };
 
-  // Staging of an E tile: thread t holds rows t/32 + 8q, chunk t % 32.
-  f4 stage[16];
-  const bool aligned = ((p.lda * (int64_t)sizeof(float)) % 16 == 0) && (reinterpret_cast<uintptr_t>(p.lu) % 16 == 0);
+  vec_t stage[NV];
+  const bool aligned = ((p.lda * (int64_t)sizeof(T)) % 16 == 0) && (reinterpret_cast<uintptr_t>(p.lu) % 16 == 0);
   auto fetch = [&](int cb) {
-    const int cc = (t & 31) * 4;
+    const int rb0 = TRANS ? cb : r0, cb0 = TRANS ? r0 : cb;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int grow = r0 + (t >> 5) + 8 * q, gcol = cb + cc;
-      if (aligned && grow < p.n && gcol + 4 <= p.n) {
-        stage[q] = *reinterpret_cast<const f4 *>(p.lu + (int64_t)grow * p.lda + gcol);
+    for (int q = 0; q < NV; ++q) {
+      const int lin = (q * 256 + t) * VEC, grow = rb0 + lin / BS, gcol = cb0 + lin % BS;
+      if (aligned && grow < p.n && gcol + VEC <= p.n) {
+        stage[q] = *reinterpret_cast<const vec_t *>(p.lu + (int64_t)grow * p.lda + gcol);
       } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          stage[q][e] = (grow < p.n && gcol + e < p.n) ? p.lu[(int64_t)grow * p.lda + gcol + e] : 0.0f;
+        for (int e = 0; e < VEC; ++e)
+          stage[q][e] = (grow < p.n && gcol + e < p.n) ? p.lu[(int64_t)grow * p.lda + gcol + e] : T(0);
       }
     }
   };
   auto stash = [&]() {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) *reinterpret_cast<f4 *>(tile + swz((t >> 5) + 8 * q, t & 31)) = stage[q];
+    for (int q = 0; q < NV; ++q) {
+      const int lin = (q * 256 + t) * VEC;
+      *reinterpret_cast<vec_t *>(tile + lin / BS * P + lin % BS) = stage[q];
+    }
+  };
+  // Four consecutive k of row `row` of E, of column lc of the second operand.
+  auto a_of = [&](int row, int k) -> v4 {
+    v4 v;
+    if (TRANS) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = tile[(k + e) * P + row];
+    } else {
+      __builtin_memcpy(&v, __builtin_assume_aligned(tile + row * P + k, 16), sizeof v);
+    }
+    return v;
+  };
+  auto b_of = [&](int k) -> v4 {
+    v4 v;
+    __builtin_memcpy(&v, __builtin_assume_aligned(&xs[lc][k], 16), sizeof v);
+    return v;
   };
 
-  // D_i^-1 in the MFMA A-operand layout: dreg[rb][s] = D[row(rb)][16 s + 4 g .. + 3].
-  f4 dreg[2][8];
+  // D_i^-1 in the first operand's layout.
+  v4 dreg[RB][KS];
   {
-    const float *D = p.dinv + (size_t)i * BS * BS;
+    const T *D = p.dinv + (size_t)i * BS * BS;
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-      for (int s = 0; s < 8; ++s)
-        dreg[rb][s] = *reinterpret_cast<const f4 *>(D + (32 * wave + 16 * rb + lc) * BS + 16 * s + 4 * g);
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int row = wrow + 16 * rb + lc, k = 16 * s + 4 * g + e;
+          dreg[rb][s][e] = TRANS ? D[k * BS + row] : D[row * BS + k];
+        }
   }
-  f4 acc[2];
+  v4 acc[RB];
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
+  for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int gi = r0 + arow(rb, r);
-      acc[rb][r] = (gi < p.n && lc < ncols) ? p.xin[(int64_t)gi * p.ldx + c0 + lc] : 0.0f;
+      acc[rb][r] = (gi < p.n && lc < ncols) ? p.xin[(int64_t)gi * p.ldx + c0 + lc] : T(0);
     }
   if (t == 0) s_bail = 0;
 
@@ -1246,36 +1300,37 @@ __global__ void __launch_bounds__(256, 2) trsm_mfma_kernel(TrsvArgs<float> p) {
     __syncthreads();  // the previous product is done with tile and xs
     stash();
     if (d + 1 < nb) fetch(dep(d + 1) * BS);
-    // The solved values of block j: every thread polls its own tagged words
-    // (bounded waits).
+    // The solved values of block j: word `part` (the high one first) of
+    // element (kr, q).  Past the matrix the last row's words stand in.
     {
+      unsigned long long w[NWD];
       bool bail = false;
-#pragma unroll
-      for (int e0 = 0; e0 < BS * RC; e0 += 256) {
-        const int e = e0 + t, kr = e / RC, q = e % RC;
-        const int gi = cb + kr;
-        float v = 0.0f;
-        if (gi < p.n && q < ncols) {
-          const unsigned long long *w = p.xt + ((int64_t)gi * p.nrhs + c0 + q);
-          int spins = 0;
-          for (;;) {
-            if (spins >= p.wait_limit) {
-              bail = true;
-              break;
-            }
-            const unsigned long long x = ld_sc1(w);
-            if ((uint32_t)(x >> 32) == p.epoch) {
-              v = __uint_as_float((uint32_t)x);
-              break;
-            }
-            if ((++spins & 63) == 0 && ld_sc1(p.err) != 0) {
-              bail = true;
-              break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-          }
+      for (int spins = 0;;) {
+        bool ok = spins < p.wait_limit;
+        if (!ok) {
+          bail = true;
+          break;
         }
-        xs[q][kr] = -v;
+#pragma unroll
+        for (int m = 0; m < NWD; ++m) {
+          const int e = m * 256 + t, kr = e / (RC * WPE), q = e % (RC * WPE) / WPE, part = e % WPE;
+          const int gi = min(cb + kr, p.n - 1), gq = c0 + min(q, ncols - 1);
+          w[m] = ld_sc1(p.xt + ((int64_t)gi * p.nrhs + gq) * WPE + part);
+        }
+#pragma unroll
+        for (int m = 0; m < NWD; ++m) ok = ok && (uint32_t)(w[m] >> 32) == p.epoch;
+        if (ok) break;
+        if ((++spins & 63) == 0 && ld_sc1(p.err) != 0) {
+          bail = true;
+          break;
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < NWD; ++m) {
+        const int e = m * 256 + t, kr = e / (RC * WPE), q = e % (RC * WPE) / WPE, part = e % WPE;
+        uint32_t x = cb + kr < p.n ? (uint32_t)w[m] : 0u;
+        x ^= part == 0 ? 0x80000000u : 0u;  // -X_j
+        reinterpret_cast<uint32_t *>(&xs[q][kr])[WPE - 1 - part] = x;
       }
       if (bail) {
         atomic_or_agent(p.err, kErrWait);
@@ -1285,43 +1340,59 @@ __global__ void __launch_bounds__(256, 2) trsm_mfma_kernel(TrsvArgs<float> p) {
     __syncthreads();
     if (s_bail) return;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const f4 bq = *reinterpret_cast<const f4 *>(&xs[lc][16 * s + 4 * g]);
+    for (int rb = 0; rb < RB; ++rb) {
+      v4 sum[NC];
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
-        const f4 aq = *reinterpret_cast<const f4 *>(tile + swz(32 * wave + 16 * rb + lc, 4 * s + g));
+      for (int s = 0; s < KS; ++s) {
+        const v4 bq = b_of(16 * s + 4 * g);
+        const v4 aq = a_of(wrow + 16 * rb + lc, 16 * s + 4 * g);
+        if (s < NC) sum[s] = v4{T(0), T(0), T(0), T(0)};
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) acc[rb] = __builtin_amdgcn_mfma_f32_16x16x4f32(aq[ks], bq[ks], acc[rb], 0, 0, 0);
+        for (int ks = 0; ks < 4; ++ks) sum[s % NC] = M::op(aq[ks], bq[ks], sum[s % NC]);
       }
+#pragma unroll
+      for (int w = NC / 2; w >= 1; w /= 2)
+#pragma unroll
+        for (int q = 0; q < w; ++q) sum[q] += sum[q + w];
+      acc[rb] += sum[0];
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
   __syncthreads();  // the last product is done with xs
-  // y (this block's right-hand sides minus the dependencies) as the B operand.
+  // y (this block's right-hand sides minus the dependencies) as the second operand.
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
+  for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
     for (int r = 0; r < 4; ++r) xs[lc][arow(rb, r)] = acc[rb][r];
   __syncthreads();
-  f4 out[2];
+  v4 out[RB];
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb) out[rb] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+  for (int rb = 0; rb < RB; ++rb) {
+    v4 sum[NC];
 #pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    const f4 bq = *reinterpret_cast<const f4 *>(&xs[lc][16 * s + 4 * g]);
+    for (int s = 0; s < KS; ++s) {
+      const v4 bq = b_of(16 * s + 4 * g);
+      if (s < NC) sum[s] = v4{T(0), T(0), T(0), T(0)};
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+      for (int ks = 0; ks < 4; ++ks) sum[s % NC] = M::op(dreg[rb][s][ks], bq[ks], sum[s % NC]);
+    }
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
-        out[rb] = __builtin_amdgcn_mfma_f32_16x16x4f32(dreg[rb][s][ks], bq[ks], out[rb], 0, 0, 0);
+    for (int w = NC / 2; w >= 1; w /= 2)
+#pragma unroll
+      for (int q = 0; q < w; ++q) sum[q] += sum[q + w];
+    out[rb] = sum[0];
+    __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
+  for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int gi = r0 + arow(rb, r);
       if (gi < p.n && lc < ncols) {
+        unsigned long long *w = p.xt + ((int64_t)gi * p.nrhs + c0 + lc) * WPE;
+#pragma unroll
+        for (int k = 0; k < WPE; ++k) st_sc1(w + k, tagged(p.epoch, word_of<T>(out[rb][r], k)));
         p.x[(int64_t)gi * p.ldx + c0 + lc] = out[rb][r];
-        st_sc1(p.xt + ((int64_t)gi * p.nrhs + c0 + lc), tagged(p.epoch, __float_as_uint(out[rb][r])));
       }
     }
 }
@@ -1332,11 +1403,14 @@ static hipError_t trsv_launch(lair_context *ctx, const T *lu, int64_t lda, const
                               bool forward, bool trans, IrFuse *fz) {
   if (n <= 0 || nrhs <= 0) return hipSuccess;
   constexpr int BS = TrsvBlock<T>::BS;
-  // Right-hand sides per workgroup: 4 columns keep each chain link short
-  // (the link's products and reductions grow with the chunk width), and the
-  // chunks run as independent chains.  FP32 with 16 or more right-hand sides
-  // (not transposed) runs the matrix-core kernel in chunks of 16.
-  const bool mfma = std::is_same<T, float>::value && nrhs >= 16 && !trans && !dinv_trans;
+  // From two right-hand sides on the matrix cores win over the vector kernel
+  // (64-row blocks, chunks of 4), both solves of n = 4096 in FP64: 378 against
+  // 569 us at 2, 373 against 667 at 4, 422 against 1027 at 16, 471 against
+  // 1550 at 40; n = 300: 67 against 77 us at 2.  One right-hand side stays
+  // with the vector kernel (285 us: no operand staging in its chain links).
+  // The fused refinement step has its own kernel, in chunks of 4.
+  const bool mfma = !fz && nrhs > 1;
+  if (mfma && trans != dinv_trans) return hipErrorInvalidValue;
   const int rc = mfma ? 16 : (nrhs == 1 ? 1 : 4);
   const int nblk = (n + BS - 1) / BS;
   const int nchunks = (nrhs + rc - 1) / rc;
@@ -1382,8 +1456,7 @@ static hipError_t trsv_launch(lair_context *ctx, const T *lu, int64_t lda, const
   a.wait_limit = ctx->wait_limit;
   const unsigned grid = (unsigned)(nblk * nchunks);
   const size_t shm = (size_t)BS * (BS + 16 / sizeof(T)) * sizeof(T);
-  static bool once = (allow_large_lds(trsv_dataflow_kernel<T, BS, 1>),
-                      allow_large_lds(trsv_dataflow_kernel<T, BS, 4>), true);
+  static bool once = (allow_large_lds(trsv_dataflow_kernel<T, BS>), true);
   (void)once;
   if constexpr (std::is_same<T, float>::value) {
     if (fz) {
@@ -1405,20 +1478,19 @@ static hipError_t trsv_launch(lair_context *ctx, const T *lu, int64_t lda, const
     }
   }
   const int slot = prof_begin(ctx, LAIR_KCLASS_GETRS);
-  if constexpr (std::is_same<T, float>::value) {
-    if (mfma) {
-      static bool once_m = (allow_large_lds(trsm_mfma_kernel), true);
-      (void)once_m;
-      trsm_mfma_kernel<<<grid, 256, (size_t)BS * BS * sizeof(float), ctx->stream>>>(a);
-      prof_end(ctx, slot, LAIR_KCLASS_GETRS, (double)n * n * nrhs,
-               sizeof(T) * (0.5 * (double)n * n + 2.0 * n * nrhs));
-      return hipGetLastError();
-    }
+  if (mfma) {
+    static bool once_m = (allow_large_lds(trsm_mfma_kernel<T, BS, false>),
+                          allow_large_lds(trsm_mfma_kernel<T, BS, true>), true);
+    (void)once_m;
+    if (trans)
+      trsm_mfma_kernel<T, BS, true><<<grid, 256, shm, ctx->stream>>>(a);
+    else
+      trsm_mfma_kernel<T, BS, false><<<grid, 256, shm, ctx->stream>>>(a);
+    prof_end(ctx, slot, LAIR_KCLASS_GETRS, (double)n * n * nrhs,
+             sizeof(T) * (0.5 * (double)n * n + 2.0 * n * nrhs));
+    return hipGetLastError();
   }
-  if (rc == 1)
-    trsv_dataflow_kernel<T, BS, 1><<<grid, 256, shm, ctx->stream>>>(a);
-  else
-    trsv_dataflow_kernel<T, BS, 4><<<grid, 256, shm, ctx->stream>>>(a);
+  trsv_dataflow_kernel<T, BS><<<grid, 256, shm, ctx->stream>>>(a);
   prof_end(ctx, slot, LAIR_KCLASS_GETRS, (double)n * n * nrhs,
            sizeof(T) * (0.5 * (double)n * n + 2.0 * n * nrhs));
   return hipGetLastError();
