@@ -66,7 +66,7 @@ def gen_lib():
 
 def bench_batched(ctx, gl, dtype, steps, count=20000, seed=4):
     """C4: `count` systems, n ~ U{8..256}, A ~ N(0,1) + n I, nrhs ~ U{1,2,4},
-    solved in one graph-captured persistent launch (plan autotuned once).
+    solved in one graph of a launch per size class.
     Inputs are regenerated on the device before every timed launch (untimed)."""
     import lair_amd as L
     rng = np.random.default_rng(seed)

@@ -273,10 +273,10 @@ lair_status lair_dbackward_error(lair_context *ctx, int64_t n, int64_t nrhs, con
  * sum_{j<i} n_j of `ipiv`; info[i] = -1 or the last zero-pivot column.
  * a is overwritten by the LU factors and b by X.  precision: 0 = FP64,
  * 1 = FP32 (a, b are float).  The plan sorts the systems by decreasing n,
- * optionally autotunes (flags & LAIR_BATCHED_AUTOTUNE: the systems may be
- * split into two size classes, and each class's launch shape is chosen by
- * timing candidates on scratch copies of a and b) and captures the launches
- * in one hipGraph on the context's stream. */
+ * splits them into size classes (n <= 64, 128, 256: one, two, four waves per
+ * system) and captures the classes' launches in one hipGraph that runs on the
+ * context's stream.  LAIR_BATCHED_AUTOTUNE is accepted in flags; the launch
+ * shape follows from the sizes and nothing has to be timed. */
 #define LAIR_BATCHED_AUTOTUNE 1
 typedef struct lair_batched_plan lair_batched_plan;
 lair_status lair_gesv_batched_plan(lair_context *ctx, int32_t precision, int32_t count,
@@ -285,8 +285,8 @@ lair_status lair_gesv_batched_plan(lair_context *ctx, int32_t precision, int32_t
                                    lair_batched_plan **plan);
 /* Replays the captured graph (asynchronous on the context's stream). */
 lair_status lair_gesv_batched_run(lair_batched_plan *plan);
-/* Launch shape chosen for the largest systems: panel width, workgroups, LDS
- * budget (elements). */
+/* Launch shape of the largest systems: panel width, workgroups, LDS budget
+ * for whole systems (elements; 0: systems are solved in their buffers). */
 lair_status lair_gesv_batched_config(lair_batched_plan *plan, int32_t *nb, int32_t *grid,
                                      int32_t *lds_elems);
 lair_status lair_gesv_batched_destroy(lair_batched_plan *plan);

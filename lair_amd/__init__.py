@@ -175,8 +175,8 @@ def gesv_mixed(a, b, precision="fp32", max_iter=30, tol=0.0, tournament=False):
 
 
 class BatchedPlan:
-    """Plan for solving many small systems A_i X_i = B_i in one persistent,
-    graph-captured launch (packed device layout of include/lair_dev.h).
+    """Plan for solving many small systems A_i X_i = B_i in one captured graph
+    (packed device layout of include/lair_dev.h).
 
     ``a``, ``b``, ``ipiv`` and ``info`` are DeviceArray buffers holding the
     packed systems; ``run()`` overwrites a with the LU factors and b with X."""

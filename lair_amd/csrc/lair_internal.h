@@ -319,23 +319,16 @@ hipError_t launch_bgemm_tile(lair_context *ctx, int ns, int M, int N, int K, con
 // Persistent batched solver (batched.hip): device metadata and launch shape.
 struct BatchLaunch {
   int count = 0;
+  int nmax = 0;           // largest order of the launch
   const int *n = nullptr;
   const int *nrhs = nullptr;
   const int64_t *a_off = nullptr;
   const int64_t *b_off = nullptr;
   const int64_t *p_off = nullptr;
   const int *order = nullptr;
-  int *queue = nullptr;
-  int lds_max_elems = 0;  // largest augmented matrix solved in LDS
-  int nb = 16;            // panel width (8 or 16)
-  int grid = 256;         // persistent workgroups
-  int occ = 1;            // register budget for this many waves per SIMD (1: the compiler's choice)
 };
 template <typename T>
-hipError_t launch_batched_gesv(lair_context *ctx, const BatchLaunch &bl, T *a, T *b, int64_t *ipiv,
-                               int *info);
-size_t batched_lds_bytes_for(int elem_size, int nb, int lds_max_elems);
-void batched_prepare();
+hipError_t launch_batched_gesv(const BatchLaunch &bl, T *a, T *b, int64_t *ipiv, int *info, hipStream_t stream);
 
 // Copies nw words and the status word to ctx->pub_dev[2..] and [1], then
 // writes seq to ctx->pub_dev[0] (system-scope release) for the host to poll.

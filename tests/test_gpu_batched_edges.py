@@ -1,0 +1,99 @@
+"""The batched solver where its blocks, panels and size classes end: orders at
+and around 16 (a register panel), 32 (a block), 64 and 128 (one, two, four
+waves), matrices without a dominant diagonal (every column interchanges rows,
+within and below the block), equal magnitudes, zero columns, and entries near
+the end of the exponent range (where the back substitution divides instead of
+multiplying by a reciprocal).
+
+Pivots and zero-pivot columns have to equal those of the reference's row-major
+LU (the oracle); the backward error |b - A x| / (|A| |x|) is within 8 n eps: n
+rounded products per unknown in each of the factorization and the two
+substitutions, and the growth of the pivots of a random matrix of these orders
+(below 8).
+"""
+import numpy as np
+import pytest
+
+import lair_amd as L
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+ORDERS = [1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 63, 64, 65, 96, 127, 128, 129, 160, 191, 225, 255, 256]
+
+
+def _run(As, Bs, dtype):
+    ns = np.array([len(A) for A in As], np.int32)
+    rs = np.array([B.shape[1] for B in Bs], np.int32)
+    da = L.DeviceArray.from_host(np.concatenate([A.ravel() for A in As]).reshape(-1, 1))
+    db = L.DeviceArray.from_host(np.concatenate([B.ravel() for B in Bs]).reshape(-1, 1))
+    dp = L.DeviceArray(int(ns.sum()), 1, np.int64)
+    di = L.DeviceArray(len(ns), 1, np.int32)
+    ctx = L.Context()
+    plan = L.BatchedPlan(ctx, ns, rs, da, db, dp, di, precision=0 if dtype == np.float64 else 1)
+    plan.run()
+    ctx.synchronize()
+    lu, x, piv, info = (d.download().ravel() for d in (da, db, dp, di))
+    plan.close()
+    for d in (da, db, dp, di):
+        d.free()
+    ctx.close()
+    oa, ob, op = (np.concatenate([[0], np.cumsum(k)]) for k in (ns * ns, ns * rs, ns))
+    return [(lu[oa[i]:oa[i + 1]].reshape(n, n), x[ob[i]:ob[i + 1]].reshape(n, -1), piv[op[i]:op[i + 1]], info[i])
+            for i, n in enumerate(ns)]
+
+
+def _oracle(A):
+    ref = A.copy()
+    piv, sing = O.getrf(ref) if A.dtype == np.float64 else O.sgetrf(ref)
+    return ref, piv, -1 if sing is None else sing
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("scale", [0, 1])
+def test_orders_and_interchanges(dtype, scale):
+    rng = np.random.default_rng(97)
+    e = scale * (1005 if dtype == np.float64 else 110)
+    As = [np.ldexp(rng.standard_normal((n, n)), e).astype(dtype) for n in ORDERS]
+    Bs = [np.ldexp(rng.standard_normal((n, r)), e).astype(dtype) for n, r in zip(ORDERS, [1, 4, 5, 16] * 6)]
+    eps = float(np.finfo(dtype).eps)
+    for A, B, (lu, x, piv, info) in zip(As, Bs, _run(As, Bs, dtype)):
+        n = len(A)
+        ref, piv_o, sing_o = _oracle(A)
+        assert info == sing_o == -1
+        np.testing.assert_array_equal(piv, piv_o, err_msg=f"n={n}")
+        a64, b64, x64 = np.ldexp(A.astype(np.float64), -e), np.ldexp(B.astype(np.float64), -e), x.astype(np.float64)
+        assert np.abs(b64 - a64 @ x64).max() <= 8 * n * eps * np.abs(a64).sum(1).max() * np.abs(x64).max(), n
+        # The factors reproduce the interchanged matrix (the columns of L got
+        # every later interchange).
+        l64, u64 = np.tril(lu.astype(np.float64), -1) + np.eye(n), np.triu(np.ldexp(lu.astype(np.float64), -e))
+        pa = a64.copy()
+        for i, q in enumerate(piv):
+            pa[[i, q]] = pa[[q, i]]
+        assert np.abs(l64 @ u64 - pa).max() <= 8 * n * eps * np.abs(a64).max(), n
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_ties_and_zero_columns(dtype):
+    rng = np.random.default_rng(98)
+    As, Bs = [], []
+    for n in (20, 64, 100, 130, 256):
+        A = rng.standard_normal((n, n)).astype(dtype)
+        A[:, 0] = np.where(rng.random(n) < 0.5, 2.0, -2.0)  # equal magnitudes over every wave
+        A[: n // 2, 0] = 0.5
+        As.append(A)
+        Z = rng.standard_normal((n, n)).astype(dtype)
+        Z[:, 7] = 0.0
+        Z[:, n - 3] = 0.0
+        As.append(Z)
+        N = rng.standard_normal((n, n)).astype(dtype)
+        N[3, 0] = np.nan  # never chosen
+        As.append(N)
+        Bs += [rng.standard_normal((n, 2)).astype(dtype) for _ in range(3)]
+    for i, (A, (lu, x, piv, info)) in enumerate(zip(As, _run(As, Bs, dtype))):
+        if i % 3 == 2:
+            assert piv[0] == _oracle(A)[1][0]
+            continue
+        _, piv_o, sing_o = _oracle(A)
+        np.testing.assert_array_equal(piv, piv_o, err_msg=f"{i} n={len(A)}")
+        assert info == sing_o
