@@ -13,21 +13,14 @@
 // update disjoint column ranges of the same panel, never share a slot.
 //
 // getrs (src/lapack/getrs.rs:12-39): x = P b; unit-lower forward
-// substitution x[i] -= a[i][k] x[k] for k < i in increasing k; back
-// substitution x[i] -= a[i][k] x[k] for k > i in increasing k, then
-// x[i] /= a[i][i] (num-complex DivAssign).  One workgroup per right-hand
-// side; rows i = t + 1024 s live in registers of thread t.  The forward pass
-// goes by 64-row blocks: the wave owning the block solves it (each row's
-// subtractions in increasing k), the block's values go through LDS and every
-// row below subtracts the block's 64 terms in increasing k, so each row sees
-// exactly the reference's sequence of operations.  The back substitution
-// takes its terms in increasing k, which needs every later unknown first: for
-// n <= kExactOrderMax one wave runs it row by row in that order (bit-identical
-// to the reference); beyond, the same 64-row blocking runs bottom-up (the
-// terms of a row come in decreasing block order: a backward-stable reordering
-// of the sums).
+// substitution x[i] -= a[i][k] x[k] for k < i; back substitution
+// x[i] -= a[i][k] x[k] for k > i, then x[i] /= a[i][i].  For n <=
+// kExactOrderMax one workgroup per right-hand side runs the reference's
+// operations in its order (bit-identical, num-complex DivAssign included);
+// beyond, both substitutions are dataflow solves over 64-row blocks.
 #include <algorithm>
 
+#include "device_util.h"
 #include "lair_internal.h"
 
 namespace lair {
@@ -64,171 +57,255 @@ hipError_t launch_cgemm_minus(lair_context *ctx, int mode, int M, int N, int K, 
                               reinterpret_cast<R *>(C), 2 * ldc, kclass);
 }
 
-template <typename T, int RPT>
-__global__ void __launch_bounds__(1024)
-    cgetrs_kernel(int n, const T *__restrict__ lu, int64_t lda, const int *__restrict__ perm, T *__restrict__ b,
-                  int64_t ldb) {
+// n <= kExactOrderMax, thread t keeps row t.  The forward pass goes by 64-row
+// blocks: the wave owning the block solves it (each row's subtractions in
+// increasing k), the block's values go through LDS and the rows below subtract
+// its 64 terms in increasing k.  The back substitution takes its terms in
+// increasing k, which needs every later unknown first: one wave runs it row by
+// row.
+template <typename T>
+__global__ void __launch_bounds__(kExactOrderMax)
+    cgetrs_exact_kernel(int n, const T *__restrict__ lu, int64_t lda, const int *__restrict__ perm, T *__restrict__ b,
+                        int64_t ldb) {
 #pragma clang fp contract(off)
-  constexpr int NT = 1024;
-  constexpr int LB = RPT >= 16 ? 4 : 8;  // loads in flight per batch
+  constexpr int LB = 8;  // loads in flight per batch
   __shared__ T xs[64];
   __shared__ T xall[kExactOrderMax];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int r = blockIdx.x;
-  T x[RPT];
-#pragma unroll
-  for (int s = 0; s < RPT; ++s) {
-    const int i = t + NT * s;
-    x[s] = i < n ? b[(int64_t)perm[i] * ldb + r] : T(0);
-  }
+  T x = t < n ? b[(int64_t)perm[t] * ldb + r] : T(0);
   const int nblk = (n + 63) / 64;
 
   // Forward substitution with unit lower L.
   for (int bk = 0; bk < nblk; ++bk) {
     const int k0 = bk * 64, kn = min(64, n - k0);
-    if (wave == bk % 16) {
-      const int os = k0 / NT;
+    if (wave == bk) {
+      const T *li = lu + (int64_t)(lane < kn ? k0 + lane : k0) * lda + k0;
+      for (int kc = 0; kc < kn; kc += LB) {
+        T lv[LB];
 #pragma unroll
-      for (int s = 0; s < RPT; ++s) {
-        if (s == os) {
-          const int i = k0 + lane;
-          const T *li = lu + (int64_t)(lane < kn ? i : k0) * lda + k0;
-          T xv = x[s];
-          for (int kc = 0; kc < kn; kc += LB) {
-            T lv[LB];
+        for (int q = 0; q < LB; ++q) lv[q] = (kc + q < lane && lane < kn) ? li[kc + q] : T(0);
 #pragma unroll
-            for (int q = 0; q < LB; ++q) lv[q] = (kc + q < lane && lane < kn) ? li[kc + q] : T(0);
-#pragma unroll
-            for (int q = 0; q < LB; ++q) {
-              const int kk = kc + q;
-              if (kk < kn) {
-                const T xk = readlane_t(xv, kk);
-                if (kk < lane && lane < kn) {
-                  const T e = lv[q] * xk;
-                  xv = xv - e;
-                }
-              }
+        for (int q = 0; q < LB; ++q) {
+          const int kk = kc + q;
+          if (kk < kn) {
+            const T xk = readlane_t(x, kk);
+            if (kk < lane && lane < kn) {
+              const T e = lv[q] * xk;
+              x = x - e;
             }
           }
-          x[s] = xv;
-          if (lane < kn) xs[lane] = xv;
         }
       }
+      if (lane < kn) xs[lane] = x;
     }
     __syncthreads();
+    if (t >= k0 + kn && t < n) {
+      const T *li = lu + (int64_t)t * lda + k0;
+      for (int kc = 0; kc < kn; kc += LB) {
+        T lv[LB];
 #pragma unroll
-    for (int s = 0; s < RPT; ++s) {
-      const int i = t + NT * s;
-      if (i >= k0 + kn && i < n) {
-        const T *li = lu + (int64_t)i * lda + k0;
-        T xv = x[s];
-        for (int kc = 0; kc < kn; kc += LB) {
-          T lv[LB];
+        for (int q = 0; q < LB; ++q) lv[q] = kc + q < kn ? li[kc + q] : T(0);
 #pragma unroll
-          for (int q = 0; q < LB; ++q) lv[q] = kc + q < kn ? li[kc + q] : T(0);
-#pragma unroll
-          for (int q = 0; q < LB; ++q) {
-            if (kc + q < kn) {
-              const T e = lv[q] * xs[kc + q];
-              xv = xv - e;
-            }
+        for (int q = 0; q < LB; ++q) {
+          if (kc + q < kn) {
+            const T e = lv[q] * xs[kc + q];
+            x = x - e;
           }
         }
-        x[s] = xv;
       }
     }
     __syncthreads();
   }
 
   // Back substitution with U.
-  if (n <= kExactOrderMax) {
-    if (t < n) xall[t] = x[0];
-    __syncthreads();
-    if (wave == 0) {
-      for (int i = n - 1; i >= 0; --i) {
-        const T *ui = lu + (int64_t)i * lda;
-        const int c0 = i + 1 + lane, c1 = i + 65 + lane;
-        const T u0 = c0 < n ? ui[c0] : T(0);
-        const T u1 = c1 < n ? ui[c1] : T(0);
-        T xi = xall[i];
-        for (int k = i + 1; k < n; ++k) {
-          const int q = k - i - 1;
-          const T u = q < 64 ? readlane_t(u0, q) : readlane_t(u1, q - 64);
-          const T e = u * xall[k];
-          xi = xi - e;
-        }
-        const T xn = cplx_div(xi, ui[i]);
-        if (lane == 0) xall[i] = xn;
+  if (t < n) xall[t] = x;
+  __syncthreads();
+  if (wave == 0) {
+    for (int i = n - 1; i >= 0; --i) {
+      const T *ui = lu + (int64_t)i * lda;
+      const int c0 = i + 1 + lane, c1 = i + 65 + lane;
+      const T u0 = c0 < n ? ui[c0] : T(0);
+      const T u1 = c1 < n ? ui[c1] : T(0);
+      T xi = xall[i];
+      for (int k = i + 1; k < n; ++k) {
+        const int q = k - i - 1;
+        const T u = q < 64 ? readlane_t(u0, q) : readlane_t(u1, q - 64);
+        const T e = u * xall[k];
+        xi = xi - e;
       }
-    }
-    __syncthreads();
-    if (t < n) x[0] = xall[t];
-  } else {
-    for (int bk = nblk - 1; bk >= 0; --bk) {
-      const int k0 = bk * 64, kn = min(64, n - k0);
-      if (wave == bk % 16) {
-        const int os = k0 / NT;
-#pragma unroll
-        for (int s = 0; s < RPT; ++s) {
-          if (s == os) {
-            const int i = k0 + lane;
-            const T *ui = lu + (int64_t)(lane < kn ? i : k0) * lda + k0;
-            const T dii = lane < kn ? ui[lane] : T(1);
-            T xv = x[s];
-            for (int kc = kn - 1; kc >= 0; kc -= LB) {
-              T uv[LB];
-#pragma unroll
-              for (int q = 0; q < LB; ++q) {
-                const int kk = kc - q;
-                uv[q] = (kk >= 0 && kk > lane && lane < kn) ? ui[kk] : T(0);
-              }
-#pragma unroll
-              for (int q = 0; q < LB; ++q) {
-                const int kk = kc - q;
-                if (kk >= 0) {
-                  if (lane == kk) xv = cplx_div(xv, dii);
-                  const T xk = readlane_t(xv, kk);
-                  if (lane < kk) {
-                    const T e = uv[q] * xk;
-                    xv = xv - e;
-                  }
-                }
-              }
-            }
-            x[s] = xv;
-            if (lane < kn) xs[lane] = xv;
-          }
-        }
-      }
-      __syncthreads();
-#pragma unroll
-      for (int s = 0; s < RPT; ++s) {
-        const int i = t + NT * s;
-        if (i < k0) {
-          const T *ui = lu + (int64_t)i * lda + k0;
-          T xv = x[s];
-          for (int kc = 0; kc < kn; kc += LB) {
-            T uv[LB];
-#pragma unroll
-            for (int q = 0; q < LB; ++q) uv[q] = kc + q < kn ? ui[kc + q] : T(0);
-#pragma unroll
-            for (int q = 0; q < LB; ++q) {
-              if (kc + q < kn) {
-                const T e = uv[q] * xs[kc + q];
-                xv = xv - e;
-              }
-            }
-          }
-          x[s] = xv;
-        }
-      }
-      __syncthreads();
+      const T xn = cplx_div(xi, ui[i]);
+      if (lane == 0) xall[i] = xn;
     }
   }
+  __syncthreads();
+  if (t < n) b[(int64_t)t * ldb + r] = xall[t];
+}
+
+// acc - a b, by fused multiply-adds.
+template <typename R>
+__device__ __forceinline__ cplx<R> csub_mul(cplx<R> acc, cplx<R> a, cplx<R> b) {
+  return cplx<R>(__builtin_elementwise_fma(a.im, b.im, __builtin_elementwise_fma(-a.re, b.re, acc.re)),
+                 __builtin_elementwise_fma(-a.im, b.re, __builtin_elementwise_fma(-a.re, b.im, acc.im)));
+}
+
+// c ? a : b by components (a conditional on the struct goes through memory).
+template <typename R>
+__device__ __forceinline__ cplx<R> csel(bool c, cplx<R> a, cplx<R> b) {
+  return cplx<R>(c ? a.re : b.re, c ? a.im : b.im);
+}
+
+// n > kExactOrderMax: one substitution (unit lower forward, or upper backward)
+// as a dataflow.  Workgroup (block row i of 64 rows, right-hand side) has four
+// threads per row subtract E_ij x_j, 16 columns each, for the blocks j solved
+// before it (their E entries are requested before the wait for x_j), then one
+// wave solves the diagonal block by substitution, a lane per row, from the
+// block's transpose in LDS, and publishes its values as tagged words.  Blocks
+// start in the order of the solve, so every wait ends; waits are bounded.
+//
+// The quotients of the back substitution are x conj(d) / |d|^2 by the
+// precomputed inverse of d and one correction by the remainder, which is at
+// least as close as the direct formula; blocks with a diagonal entry far from
+// 1 in the exponent use the direct formula.
+//
+// Bound by the chain: 64 substitution steps per block (1.4 us with f64
+// components, 5.5 us with the quotients) and one round trip of the words.
+// n = 1500 with three right-hand sides: 109 + 209 us, where one workgroup per
+// right-hand side, a row per thread, took 1920 us.
+constexpr int kCflowBS = 64;
+template <typename T>
+struct CflowArgs {
+  const T *lu;
+  int64_t lda;
+  const int *perm;  // rows of x_in, or null
+  const T *xin;
+  int64_t ldi;
+  T *x;
+  int64_t ldx;
+  int n, nrhs, nblk;
+  unsigned long long *xt;  // [nrhs][n][words] tagged solved values
+  uint32_t epoch;
+  int32_t *err;
+  int wait_limit;
+};
+
+template <typename T, bool UPPER>
+__global__ void __launch_bounds__(256, 2) cgetrs_flow_kernel(CflowArgs<T> p) {
+  typedef typename cplx_traits<T>::real R;
+  constexpr int BS = kCflowBS, WPE = sizeof(T) / 4, H = WPE / 2, SEG = 16, LD = BS + 1;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  T *dt = reinterpret_cast<T *>(smem_raw);  // [k][row]: the diagonal block
+  __shared__ T xs[2][BS];
+  __shared__ T ys[BS];
+  __shared__ int s_bail[2];  // by block parity
+  const int t = threadIdx.x, lane = t & 63;
+  const int ib = blockIdx.x / p.nrhs, c = blockIdx.x % p.nrhs;
+  const int i = UPPER ? p.nblk - 1 - ib : ib;
+  const int r0 = i * BS, w = min(BS, p.n - r0);
+  const int r = t >> 2, h = t & 3;
+  const int gr = min(r0 + r, p.n - 1);
+  unsigned long long *xt = p.xt + (int64_t)c * p.n * WPE;
+  if (t < 2) s_bail[t] = 0;
+
+  for (int e = t; e < BS * BS; e += 256) {
+    const int row = e / BS, k = e % BS;
+    dt[k * LD + row] = p.lu[(int64_t)min(r0 + row, p.n - 1) * p.lda + min(r0 + k, p.n - 1)];
+  }
+  const T *row = p.lu + (int64_t)gr * p.lda;
+  T seg[SEG], acc(0);
+  auto dep = [&](int d) { return UPPER ? p.nblk - 1 - d : d; };
+  auto fetch = [&](int cb) {
 #pragma unroll
-  for (int s = 0; s < RPT; ++s) {
-    const int i = t + NT * s;
-    if (i < n) b[(int64_t)i * ldb + r] = x[s];
+    for (int s = 0; s < SEG; ++s) seg[s] = row[min(cb + h * SEG + s, p.n - 1)];
+  };
+  T bval(0);
+  if (h == 0) bval = p.xin[(int64_t)(p.perm ? p.perm[gr] : gr) * p.ldi + c];
+  if (ib > 0) fetch(dep(0) * BS);
+  for (int d = 0; d < ib; ++d) {
+    const int cb = dep(d) * BS;
+    T *xd = xs[d & 1];
+    // Element kr's words; past the matrix (ragged last block) zeros.
+    if (t < BS * H) {
+      const int kr = t / H, gi = min(cb + kr, p.n - 1), part = t % H;
+      const unsigned long long *wp = xt + (int64_t)gi * WPE + part;
+      unsigned long long w0, w1;
+      for (int spins = 0;;) {
+        if (spins >= p.wait_limit) {
+          atomic_or_agent(p.err, kErrWait);
+          s_bail[d & 1] = 1;
+          w0 = w1 = 0;
+          break;
+        }
+        w0 = ld_agent(wp);
+        w1 = ld_agent(wp + H);
+        if ((uint32_t)(w0 >> 32) == p.epoch && (uint32_t)(w1 >> 32) == p.epoch) break;
+        if ((++spins & 63) == 0 && ld_agent(p.err) != 0) {
+          s_bail[d & 1] = 1;
+          break;
+        }
+      }
+      // word_of: the real part's words, then the imaginary part's, high first.
+      uint32_t *dst = reinterpret_cast<uint32_t *>(&xd[kr]);
+      const bool in = cb + kr < p.n;
+      dst[H - 1 - part] = in ? (uint32_t)w0 : 0u;
+      dst[WPE - 1 - part] = in ? (uint32_t)w1 : 0u;
+    }
+    __syncthreads();
+    if (s_bail[d & 1]) return;
+#pragma unroll
+    for (int s = 0; s < SEG; ++s) acc = csub_mul(acc, seg[s], xd[h * SEG + s]);
+    if (d + 1 < ib) fetch(dep(d + 1) * BS);
+  }
+#pragma unroll
+  for (int off = 2; off >= 1; off >>= 1)
+    acc = T(acc.re + __shfl_xor(acc.re, off), acc.im + __shfl_xor(acc.im, off));
+  if (h == 0) ys[r] = r < w ? T(bval.re + acc.re, bval.im + acc.im) : T(0);
+  __syncthreads();
+  if (t >= 64) return;
+  T x = ys[lane];
+  if (!UPPER) {
+    for (int k0 = 0; k0 < w; k0 += 8) {
+      T l[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) l[q] = dt[(k0 + q) * LD + lane];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const T nx = csub_mul(x, l[q], readlane_t(x, k0 + q));
+        x = csel(lane > k0 + q && lane < w, nx, x);
+      }
+    }
+  } else {
+    const T dg = dt[lane * LD + lane];
+    const R ns = dg.re * dg.re + dg.im * dg.im;
+    const R lo = sizeof(R) == 8 ? R(0x1p-500) : R(0x1p-60f), hi = sizeof(R) == 8 ? R(0x1p500) : R(0x1p60f);
+    const bool fast = __all(lane >= w || (ns >= lo && ns <= hi));
+    const T inv(dg.re / ns, -dg.im / ns);
+    for (int k0 = (w - 1) / 8 * 8; k0 >= 0; k0 -= 8) {
+      T u[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) u[q] = dt[(k0 + q) * LD + lane];
+#pragma unroll
+      for (int q = 7; q >= 0; --q) {
+        if (k0 + q < w) {
+          T v;
+          if (fast) {
+            v = csub_mul(T(0), T(-x.re, -x.im), inv);
+            v = csub_mul(v, T(0) - csub_mul(x, v, dg), inv);
+          } else {
+            v = cplx_div(x, dg);
+          }
+          x = csel(lane == k0 + q, v, x);
+          const T nx = csub_mul(x, u[q], readlane_t(x, k0 + q));
+          x = csel(lane < k0 + q, nx, x);
+        }
+      }
+    }
+  }
+  if (lane < w) {
+    unsigned long long *wp = xt + (int64_t)(r0 + lane) * WPE;
+#pragma unroll
+    for (int k = 0; k < WPE; ++k) st_agent(wp + k, tagged(p.epoch, word_of<T>(x, k)));
+    p.x[(int64_t)(r0 + lane) * p.ldx + c] = x;
   }
 }
 
@@ -237,16 +314,56 @@ hipError_t launch_cgetrs(lair_context *ctx, int n, int nrhs, const T *lu, int64_
                          int64_t ldb) {
   if (n <= 0 || nrhs <= 0) return hipSuccess;
   if (n > kComplexGetrsMax) return hipErrorInvalidValue;
-  const int slot = prof_begin(ctx, LAIR_KCLASS_GETRS);
-  const dim3 grid(nrhs), block(1024);
   hipStream_t st = ctx->stream;
-  if (n <= 1024) cgetrs_kernel<T, 1><<<grid, block, 0, st>>>(n, lu, lda, perm, b, ldb);
-  else if (n <= 2048) cgetrs_kernel<T, 2><<<grid, block, 0, st>>>(n, lu, lda, perm, b, ldb);
-  else if (n <= 4096) cgetrs_kernel<T, 4><<<grid, block, 0, st>>>(n, lu, lda, perm, b, ldb);
-  else if (n <= 8192) cgetrs_kernel<T, 8><<<grid, block, 0, st>>>(n, lu, lda, perm, b, ldb);
-  else cgetrs_kernel<T, 16><<<grid, block, 0, st>>>(n, lu, lda, perm, b, ldb);
-  prof_end(ctx, slot, LAIR_KCLASS_GETRS, 8.0 * (double)n * n * nrhs,
-           (double)sizeof(T) * ((double)n * n * nrhs + 2.0 * n * nrhs));
+  if (n <= kExactOrderMax) {
+    const int slot = prof_begin(ctx, LAIR_KCLASS_GETRS);
+    cgetrs_exact_kernel<T><<<nrhs, kExactOrderMax, 0, st>>>(n, lu, lda, perm, b, ldb);
+    prof_end(ctx, slot, LAIR_KCLASS_GETRS, 8.0 * (double)n * n * nrhs,
+             (double)sizeof(T) * ((double)n * n * nrhs + 2.0 * n * nrhs));
+    return hipGetLastError();
+  }
+  // Passes of at most 64 right-hand sides bound the workspaces.
+  const int chunk = std::min(nrhs, 64);
+  hipError_t e = ensure(ctx->ws_tmp2, sizeof(T) * (size_t)n * chunk);
+  if (e != hipSuccess) return e;
+  CflowArgs<T> a;
+  e = tri_words(ctx, (size_t)n * chunk * (sizeof(T) / 4), &a.xt);
+  if (e != hipSuccess) return e;
+  const size_t shm = sizeof(T) * kCflowBS * (kCflowBS + 1);
+  static const hipError_t once[2] = {
+      hipFuncSetAttribute(reinterpret_cast<const void *>(cgetrs_flow_kernel<T, false>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm),
+      hipFuncSetAttribute(reinterpret_cast<const void *>(cgetrs_flow_kernel<T, true>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm)};
+  for (hipError_t o : once)
+    if (o != hipSuccess) return o;
+  a.lu = lu;
+  a.lda = lda;
+  a.n = n;
+  a.nblk = (n + kCflowBS - 1) / kCflowBS;
+  a.err = ctx->err;
+  a.wait_limit = ctx->wait_limit;
+  T *tmp = static_cast<T *>(ctx->ws_tmp2.ptr);
+  for (int c0 = 0; c0 < nrhs; c0 += chunk) {
+    a.nrhs = std::min(chunk, nrhs - c0);
+    const int slot = prof_begin(ctx, LAIR_KCLASS_GETRS);
+    a.perm = perm;
+    a.xin = b + c0;
+    a.ldi = ldb;
+    a.x = tmp;
+    a.ldx = a.nrhs;
+    a.epoch = ++ctx->tri_epoch;
+    cgetrs_flow_kernel<T, false><<<a.nblk * a.nrhs, 256, shm, st>>>(a);
+    a.perm = nullptr;
+    a.xin = tmp;
+    a.ldi = a.nrhs;
+    a.x = b + c0;
+    a.ldx = ldb;
+    a.epoch = ++ctx->tri_epoch;
+    cgetrs_flow_kernel<T, true><<<a.nblk * a.nrhs, 256, shm, st>>>(a);
+    prof_end(ctx, slot, LAIR_KCLASS_GETRS, 8.0 * (double)n * n * a.nrhs,
+             (double)sizeof(T) * ((double)n * n * a.nrhs + 2.0 * n * a.nrhs));
+  }
   return hipGetLastError();
 }
 

@@ -287,6 +287,7 @@ hipError_t launch_rowmap(lair_context *ctx, const int64_t *ipiv, int k0, int k1)
 // Inverses of the diagonal blocks (TrsvBlock<T>::BS) of L (unit) and U.
 template <typename T>
 hipError_t launch_trtri_diag(lair_context *ctx, const T *lu, int64_t lda, int n, T *linv, T *uinv);
+hipError_t tri_words(lair_context *ctx, size_t words, unsigned long long **xt);
 template <typename T>
 hipError_t launch_trsv_dataflow(lair_context *ctx, const T *lu, int64_t lda, const T *dinv,
                                 bool dinv_trans, const T *xin, T *x, int64_t ldx, int n, int nrhs,

@@ -1397,6 +1397,25 @@ __global__ void __launch_bounds__(256, 2) trsm_mfma_kernel(TrsvArgs<T> p) {
     }
 }
 
+// Tagged words of solved values; zeroed whenever they are (re)allocated or the
+// epoch would wrap, so that no stale word carries a live tag.
+hipError_t tri_words(lair_context *ctx, size_t words, unsigned long long **xt) {
+  const size_t bytes = sizeof(unsigned long long) * words;
+  const bool grow = ctx->ws_flags.bytes < bytes;
+  hipError_t e = ensure(ctx->ws_flags, bytes);
+  if (e != hipSuccess) return e;
+  if (grow) ctx->ws_flags_zeroed = 0;
+  if (ctx->ws_flags_zeroed < ctx->ws_flags.bytes || ctx->tri_epoch > 0x70000000u) {
+    e = launch_fill_u32(ctx, static_cast<uint32_t *>(ctx->ws_flags.ptr),
+                        (int64_t)(ctx->ws_flags.bytes / sizeof(uint32_t)), 0u);
+    if (e != hipSuccess) return e;
+    ctx->ws_flags_zeroed = ctx->ws_flags.bytes;
+    ctx->tri_epoch = 0;
+  }
+  *xt = static_cast<unsigned long long *>(ctx->ws_flags.ptr);
+  return hipSuccess;
+}
+
 template <typename T>
 static hipError_t trsv_launch(lair_context *ctx, const T *lu, int64_t lda, const T *dinv,
                               bool dinv_trans, const T *xin, T *x, int64_t ldx, int n, int nrhs,
@@ -1414,25 +1433,12 @@ static hipError_t trsv_launch(lair_context *ctx, const T *lu, int64_t lda, const
   const int rc = mfma ? 16 : (nrhs == 1 ? 1 : 4);
   const int nblk = (n + BS - 1) / BS;
   const int nchunks = (nrhs + rc - 1) / rc;
-  // Tagged words of the solved values; zeroed whenever they are (re)allocated
-  // or the epoch would wrap, so that no stale word carries a live tag.  A
-  // caller-provided buffer (xt_override) was zeroed by the caller.
+  // A caller-provided buffer (xt_override) was zeroed by the caller.
   unsigned long long *xt = ctx->xt_override;
   if (!xt) {
     // The fused refinement step also needs two words per value of x + d.
-    const size_t xt_bytes = sizeof(unsigned long long) * (size_t)n * nrhs * (sizeof(T) / 4 + (fz ? 2 : 0));
-    const bool grow = ctx->ws_flags.bytes < xt_bytes;
-    hipError_t e = ensure(ctx->ws_flags, xt_bytes);
+    const hipError_t e = tri_words(ctx, (size_t)n * nrhs * (sizeof(T) / 4 + (fz ? 2 : 0)), &xt);
     if (e != hipSuccess) return e;
-    if (grow) ctx->ws_flags_zeroed = 0;
-    if (ctx->ws_flags_zeroed < ctx->ws_flags.bytes || ctx->tri_epoch > 0x70000000u) {
-      e = launch_fill_u32(ctx, static_cast<uint32_t *>(ctx->ws_flags.ptr),
-                          (int64_t)(ctx->ws_flags.bytes / sizeof(uint32_t)), 0u);
-      if (e != hipSuccess) return e;
-      ctx->ws_flags_zeroed = ctx->ws_flags.bytes;
-      ctx->tri_epoch = 0;
-    }
-    xt = static_cast<unsigned long long *>(ctx->ws_flags.ptr);
   } else if (ctx->tri_epoch > 0x70000000u) {
     ctx->tri_epoch = 0;
   }
