@@ -365,10 +365,129 @@ hipError_t launch_dgemm_splitk_store(lair_context *ctx, int M, int N, int K, int
   return hipGetLastError();
 }
 
+// C -= A B for updates with few 128 x 128 tiles (the narrow updates of a
+// factorization, the last columns of a small one) and for the ragged edges of
+// larger ones, where one workgroup's matrix instructions on a 128 x 128 tile
+// (7 us at K = 64 in FP64), and not memory, set the time: tiles of 32 x 64, a
+// wave 16 x 32 of them, straight from global memory to MFMA operands (no LDS,
+// no barriers; the four waves share their lines in L1).  K goes by chunks of
+// 32, two in flight.  Step s of a chunk takes k = 16 (s / 4) + 4 g + s % 4 from
+// lane group g, so a lane's A values are contiguous.  Rows and columns past C
+// read as zero and are not written (buffer bounds); KEDGE masks a last chunk
+// that K does not fill.
+// Called alone in FP64 (20 us of call and wait included), against 128 x 128
+// tiles: 448 x 64 x 64 25 us against 54, 4000 x 64 x 64 26 / 54, 900 x 900 x
+// 128 33 / 100, 1024 x 1024 x 128 (no ragged edge) 33 / 45.
+constexpr int kSmM = 32, kSmN = 64, kSmK = 32;
+template <typename T, bool KEDGE>
+__global__ void __launch_bounds__(256)
+    gemm_small_kernel(int M, int N, int K, const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb,
+                      T *__restrict__ C, int64_t ldc) {
+  typedef typename Mfma16<T>::acc_t acc_t;
+  constexpr int ES = sizeof(T);
+  constexpr int NS = kSmK / 4;            // MFMA steps of a chunk
+  constexpr int kNone = 0x7ffffff0;       // past any buffer's end
+  const int t = threadIdx.x, lane = t & 63, g = lane >> 4, lc = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int nbn = (N + kSmN - 1) / kSmN;
+  const int bm = (int)(blockIdx.x / nbn) * kSmM + (wv & 1) * 16, bn = (int)(blockIdx.x % nbn) * kSmN + (wv >> 1) * 32;
+  if (bm >= M || bn >= N) return;
+  auto rsrc = [](const T *p, int64_t rows, int64_t ld, int64_t cols) {
+    const int64_t bytes = ((rows - 1) * ld + cols) * ES;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(p), 0, (int)min(bytes, (int64_t)0x7ffffff0), kBufWord3);
+  };
+  const int mr = min(16, M - bm);
+  const __amdgpu_buffer_rsrc_t crs = rsrc(C + (int64_t)bm * ldc + bn, mr, ldc, N - bn);
+  int co[2];
+  T cv[2][4];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    co[j] = bn + 16 * j + lc < N ? (16 * j + lc) * ES : kNone;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      cv[j][r] = buf_ld<T>(crs, bn + 16 * j + lc < N ? co[j] + Mfma16<T>::row(lane, r) * (int)ldc * ES : kNone, 0);
+  }
+  struct Chunk {
+    T a[NS], b[2][NS];
+  };
+  auto load = [&](int kc, Chunk &c) {
+    const __amdgpu_buffer_rsrc_t ars = rsrc(A + (int64_t)bm * lda + kc, mr, lda, K - kc);
+    const __amdgpu_buffer_rsrc_t brs = rsrc(B + (int64_t)kc * ldb + bn, min(kSmK, K - kc), ldb, N - bn);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int k = 16 * (s / 4) + 4 * g + s % 4;
+      const bool in = !KEDGE || kc + k < K;
+      if (KEDGE) c.a[s] = buf_ld<T>(ars, in ? (lc * (int)lda + k) * ES : kNone, 0);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) c.b[j][s] = buf_ld<T>(brs, in && co[j] != kNone ? co[j] + k * (int)ldb * ES : kNone, 0);
+    }
+    if (!KEDGE) {
+#pragma unroll
+      for (int s = 0; s < NS; s += 2) {
+        const auto v = buf_ld2<T, typename Mfma16<T>::pair_t>(
+            ars, (lc * (int)lda + 16 * (s / 4) + 4 * g + s % 4) * ES, 0);
+        c.a[s] = v[0];
+        c.a[s + 1] = v[1];
+      }
+    }
+  };
+  acc_t acc[2] = {{T(0), T(0), T(0), T(0)}, {T(0), T(0), T(0), T(0)}};
+  auto mul = [&](const Chunk &c) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[j] = Mfma16<T>::op(c.a[s], c.b[j][s], acc[j]);
+  };
+  Chunk c0, c1;
+  load(0, c0);
+  for (int kc = 0; kc < K; kc += 2 * kSmK) {
+    if (kc + kSmK < K) load(kc + kSmK, c1);
+    mul(c0);
+    if (kc + 2 * kSmK < K) load(kc + 2 * kSmK, c0);
+    if (kc + kSmK < K) mul(c1);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      buf_st<T>(cv[j][r] - acc[j][r], crs, co[j] != kNone ? co[j] + Mfma16<T>::row(lane, r) * (int)ldc * ES : kNone, 0);
+}
+
+template <typename T>
+hipError_t launch_gemm_small(lair_context *ctx, int M, int N, int K, const T *A, int64_t lda, const T *B, int64_t ldb,
+                             T *C, int64_t ldc) {
+  const unsigned grid = (unsigned)(((M + kSmM - 1) / kSmM) * ((N + kSmN - 1) / kSmN));
+  if (K % kSmK == 0)
+    gemm_small_kernel<T, false><<<grid, 256, 0, ctx->stream>>>(M, N, K, A, lda, B, ldb, C, ldc);
+  else
+    gemm_small_kernel<T, true><<<grid, 256, 0, ctx->stream>>>(M, N, K, A, lda, B, ldb, C, ldc);
+  return hipGetLastError();
+}
+template hipError_t launch_gemm_small<double>(lair_context *, int, int, int, const double *, int64_t, const double *,
+                                              int64_t, double *, int64_t);
+template hipError_t launch_gemm_small<float>(lair_context *, int, int, int, const float *, int64_t, const float *,
+                                             int64_t, float *, int64_t);
+
+// Small tiles for the whole C up to 128 large ones (half of the CUs; beyond,
+// the large tiles' reuse of A and B from LDS wins): FP64 2048 x 1024 x 256 (128
+// large tiles) 57 us against 65, 2048 x 2048 x 128 (256) 58 against 52; FP32
+// 42 / 45 and 42 / 37.  Capped launches (beside a leaf) keep to their cap.
+constexpr int kSmallTiles = 128;
+template <typename T>
+bool gemm_small_fits(const lair_context *ctx, int M, int N, int64_t lda, int64_t ldb, int64_t ldc) {
+  const int64_t tiles = (int64_t)((M + kTileM - 1) / kTileM) * ((N + kTileN - 1) / kTileN);
+  const int64_t big = std::max(std::max(lda, ldb), ldc);
+  return tiles <= kSmallTiles && ctx->bulk_wg_cap <= 0 &&
+         big <= ((int64_t)1 << 31) / ((int64_t)kTileM * (int64_t)sizeof(T));
+}
+template bool gemm_small_fits<double>(const lair_context *, int, int, int64_t, int64_t, int64_t);
+template bool gemm_small_fits<float>(const lair_context *, int, int, int64_t, int64_t, int64_t);
+
 // Splits C into the region of whole tiles (unmasked kernel, launched by
-// `interior`) and the right and bottom strips (masked kernel, one tile per
-// workgroup, launched by `masked`); K not a multiple of the stage depth runs
-// masked throughout.  The 32-bit buffer offsets need 128 rows of C, A and B
+// `interior`) and the right and bottom strips (launched by `masked`: small
+// tiles where there is such a kernel, else the masked one; 4000 x 2000 x 128 in
+// FP64 with its strips: 86 against 128 us); K not a multiple of the stage depth
+// runs so throughout.  The 32-bit buffer offsets need 128 rows of C, A and B
 // within 2 GiB.
 template <typename T, bool TRANSA, typename FI, typename FM>
 static hipError_t split_tiles(int M, int N, int K, int kstep, const T *A, int64_t lda, const T *B, int64_t ldb,
@@ -390,11 +509,15 @@ static hipError_t split_tiles(int M, int N, int K, int kstep, const T *A, int64_
 template <typename T, bool TRANSA, bool STORE, typename F>
 static hipError_t gemm_split(lair_context *ctx, int M, int N, int K, const T *A, int64_t lda, const T *B,
                              int64_t ldb, T *C, int64_t ldc, F interior) {
-  hipStream_t st = ctx->stream;
+  [[maybe_unused]] hipStream_t st = ctx->stream;
   auto masked = [&](int m, int n, const T *a, const T *b, T *c) {
     if (m <= 0 || n <= 0) return;
-    const unsigned g = (unsigned)(((m + kTileM - 1) / kTileM) * ((n + kTileN - 1) / kTileN));
-    gemm_tile_kernel<T, TRANSA, STORE, 1, true><<<g, 256, 0, st>>>(m, n, K, a, lda, b, ldb, c, ldc);
+    if constexpr (!TRANSA && !STORE) {
+      (void)launch_gemm_small<T>(ctx, m, n, K, a, lda, b, ldb, c, ldc);
+    } else {
+      const unsigned g = (unsigned)(((m + kTileM - 1) / kTileM) * ((n + kTileN - 1) / kTileN));
+      gemm_tile_kernel<T, TRANSA, STORE, 1, true><<<g, 256, 0, st>>>(m, n, K, a, lda, b, ldb, c, ldc);
+    }
   };
   return split_tiles<T, TRANSA>(M, N, K, kBK, A, lda, B, ldb, C, ldc, interior, masked);
 }

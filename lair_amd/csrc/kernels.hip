@@ -944,9 +944,11 @@ hipError_t launch_gemm_minus<double>(lair_context *ctx, int mode, int M, int N, 
                                      int64_t ldb, double *C, int64_t ldc, int kclass) {
   if (M <= 0 || N <= 0 || K <= 0) return hipSuccess;
   (void)mode;
-  if (M >= 256 && N >= 32 && K >= 32) {
+  const bool small = !transA && gemm_small_fits<double>(ctx, M, N, lda, ldb, ldc);
+  if (small || (M >= 256 && N >= 32 && K >= 32)) {
     const int slot = prof_begin(ctx, kclass);
-    hipError_t e = launch_dgemm_tile(ctx, M, N, K, A, lda, transA, B, ldb, C, ldc);
+    hipError_t e = small ? launch_gemm_small<double>(ctx, M, N, K, A, lda, B, ldb, C, ldc)
+                         : launch_dgemm_tile(ctx, M, N, K, A, lda, transA, B, ldb, C, ldc);
     prof_end(ctx, slot, kclass, 2.0 * M * N * K,
              (double)sizeof(double) * (2.0 * M * N + (double)M * K + (double)K * N));
     return e;
@@ -967,10 +969,13 @@ hipError_t launch_gemm_minus<float>(lair_context *ctx, int mode, int M, int N, i
                                     const float *A, int64_t lda, bool transA, const float *B,
                                     int64_t ldb, float *C, int64_t ldc, int kclass) {
   if (M <= 0 || N <= 0 || K <= 0) return hipSuccess;
-  if (M >= 256 && N >= 32 && K >= 32 && !(transA && mode != kGemmF32)) {
+  const bool small = mode == kGemmF32 && !transA && gemm_small_fits<float>(ctx, M, N, lda, ldb, ldc);
+  if (small || (M >= 256 && N >= 32 && K >= 32 && !(transA && mode != kGemmF32))) {
     const int slot = prof_begin(ctx, kclass);
     hipError_t e;
-    if (mode == kGemmF32)
+    if (small)
+      e = launch_gemm_small<float>(ctx, M, N, K, A, lda, B, ldb, C, ldc);
+    else if (mode == kGemmF32)
       e = launch_sgemm_tile(ctx, M, N, K, A, lda, transA, B, ldb, C, ldc);
     else
       e = launch_bgemm_tile(ctx, mode == kGemmBF16x6 ? 3 : 1, M, N, K, A, lda, B, ldb, C, ldc);

@@ -304,6 +304,12 @@ hipError_t launch_trsv_ir(lair_context *ctx, const float *lu, int64_t lda, const
                           unsigned long long *rbits);
 
 // 128x128-tile MFMA trailing updates (gemm_kernels.hip).
+// C -= A B with small tiles, for a C of few large ones.
+template <typename T>
+bool gemm_small_fits(const lair_context *ctx, int M, int N, int64_t lda, int64_t ldb, int64_t ldc);
+template <typename T>
+hipError_t launch_gemm_small(lair_context *ctx, int M, int N, int K, const T *A, int64_t lda, const T *B, int64_t ldb,
+                             T *C, int64_t ldc);
 hipError_t launch_dgemm_tile(lair_context *ctx, int M, int N, int K, const double *A, int64_t lda,
                              bool transA, const double *B, int64_t ldb, double *C, int64_t ldc,
                              bool store = false);
