@@ -121,13 +121,20 @@ __device__ __forceinline__ T from_words(const uint32_t *w) {
   }
 }
 
-// Lane shuffle and read-lane of a real or complex value.
-template <typename T>
-__device__ __forceinline__ T shfl_t(T x, int src) {
+// The value of lane I of each row of 16 lanes (DPP row_newbcast), of a real or
+// complex value; read-lane likewise.
+template <int I>
+__device__ __forceinline__ int row_bcast_u32(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, 0x150 + I, 0xF, 0xF, false);
+}
+template <int I, typename T>
+__device__ __forceinline__ T row_bcast(T x) {
   if constexpr (cplx_traits<T>::is)
-    return T(__shfl(x.re, src), __shfl(x.im, src));
+    return T(row_bcast<I>(x.re), row_bcast<I>(x.im));
+  else if constexpr (sizeof(T) == 8)
+    return __hiloint2double(row_bcast_u32<I>(__double2hiint(x)), row_bcast_u32<I>(__double2loint(x)));
   else
-    return __shfl(x, src);
+    return __int_as_float(row_bcast_u32<I>(__float_as_int(x)));
 }
 template <typename R>
 __device__ __forceinline__ R readlane_real(R x, int lane) {

@@ -408,6 +408,23 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// Barrier for data in LDS only: unlike __syncthreads it does not wait for
+// global loads in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  __asm__ volatile("" ::: "memory");
+}
+
+// Steps I .. 14 of a 16-row unit lower solve, a row per lane of a row of 16.
+template <int I, typename T>
+__device__ __forceinline__ void diag_steps(T &x, const T (&lrow)[15], int rr) {
+#pragma clang fp contract(off)
+  const T e = row_bcast<I>(x) * lrow[I];
+  if (I < rr) x = x - e;
+  if constexpr (I < 14) diag_steps<I + 1>(x, lrow, rr);
+}
+
 // Interchanges then U12 = L11^-1 A12 for columns [c0, c1) of a panel
 // [k, k + kb) (kb <= 128): the laswp + trsm steps of recursive_inner
 // (src/lapack/getrf.rs:270-278) fused per 16-column strip.  The strip's rows
@@ -435,41 +452,53 @@ __global__ void __launch_bounds__(256)
   const int t = threadIdx.x;
   const int cs = c0 + blockIdx.x * CW;
   const int nc = c0 + ncols - cs < CW ? c0 + ncols - cs : CW;
+  // The row map and the first rows of L11 are requested together; the strip's
+  // rows follow as soon as the map is in LDS, while L11 still arrives.  L11
+  // goes by 256 / LW rows of LW columns per load, 32 loads at a time (its
+  // strictly lower part is kept).
   const int nr = *count;
+  const T *L = a + (int64_t)k * lda + k;
+  const int lw = kb <= 64 ? 64 : 128, lp = t & (lw - 1), lr0 = t / lw, ls = 256 / lw;
+  auto lload = [&](int r0, T (&v)[32]) {
+#pragma unroll
+    for (int q = 0; q < 32; ++q) {
+      const int r = r0 + lr0 + q * ls;
+      v[q] = (r < kb && lp < r) ? L[(int64_t)r * lda + lp] : T(0);
+    }
+  };
+  auto lstore = [&](int r0, const T (&v)[32]) {
+#pragma unroll
+    for (int q = 0; q < 32; ++q) {
+      const int r = r0 + lr0 + q * ls;
+      if (r < kb && lp < r) sL[r * (r - 1) / 2 + lp] = v[q];
+    }
+  };
   for (int e = t; e < nr; e += 256) {
     s_rows[e] = rows[e];
     s_src[e] = src[e];
   }
-  // L11 in batches of 16 independent loads per thread (the square is read,
-  // its strictly lower part kept).
-  const T *L = a + (int64_t)k * lda + k;
-  for (int b = 0; b < kb * kb; b += 256 * 16) {
-    T v[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int idx = b + q * 256 + t, r = idx / kb, p = idx % kb;
-      v[q] = (idx < kb * kb && p < r) ? L[(int64_t)r * lda + p] : T(0);
-    }
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int idx = b + q * 256 + t, r = idx / kb, p = idx % kb;
-      if (idx < kb * kb && p < r) sL[r * (r - 1) / 2 + p] = v[q];
-    }
-  }
-  __syncthreads();
+  T lv[32];
+  lload(0, lv);
+  lds_barrier();
   const int c = t % CW, rg = t / CW;
-  for (int e0 = rg; e0 < nr; e0 += RG * 16) {
+  for (int eb = 0; eb < nr; eb += RG * 16) {
+    const int e0 = eb + rg;
     T v[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
       const int e = e0 + q * RG;
       v[q] = (e < nr && c < nc) ? a[(int64_t)s_src[e] * lda + cs + c] : T(0);
     }
+    if (eb == 0) lstore(0, lv);
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
       const int e = e0 + q * RG;
       if (e < nr) sX[e * LX + c] = v[q];
     }
+  }
+  for (int r0 = 32 * ls; r0 < kb; r0 += 32 * ls) {
+    lload(r0, lv);
+    lstore(r0, lv);
   }
   __syncthreads();
   // Rows moved below the panel (entries kb.. that move something).
@@ -488,14 +517,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
       for (int i = 0; i < 15; ++i)
         lrow[i] = (i < rr && rr < bs) ? sL[(b0 + rr) * (b0 + rr - 1) / 2 + b0 + i] : T(0);
-#pragma unroll
-      for (int i = 0; i < 15; ++i) {
-        const T xi = shfl_t(x, (l & ~15) | i);
-        if (i < rr && rr < bs) {
-          const T e = xi * lrow[i];
-          x = x - e;
-        }
-      }
+      diag_steps<0>(x, lrow, rr);
       if (rr < bs) sX[(b0 + rr) * LX + cc] = x;
     }
     __syncthreads();
