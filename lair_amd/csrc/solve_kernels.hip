@@ -614,57 +614,89 @@ template hipError_t launch_trsm_llu<ccplx>(lair_context *, int, int, const ccplx
 
 // ---------------------------------------------------------- trtri_diag ---
 
+// DPP quad permutation.
+template <int CTRL, typename T>
+__device__ __forceinline__ T quad_xor(T x) {
+  if constexpr (sizeof(T) == 8)
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xF, 0xF, false),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xF, 0xF, false));
+  else
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
+}
+
 // blockIdx.x = diagonal block; blockIdx.y = 0: unit lower L -> linv,
 // 1: upper U -> uinv.  Each inverse is stored dense BS x BS (row-major).
+// Four lanes per column: each sums every fourth term of an entry's dot product
+// (four at a time, their LDS loads issued together) and the quad adds its sums
+// pairwise.  Bound by the chain of rows, a few LDS round trips each: 31 us in
+// FP64 whatever n (one lane per column, 16 loads of the block in turn: 70 us).
 template <typename T, int BS>
-__global__ void __launch_bounds__(BS)
+__global__ void __launch_bounds__(4 * BS)
     trtri_diag_kernel(const T *__restrict__ lu, int64_t lda, int n, T *__restrict__ linv,
                       T *__restrict__ uinv) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *M = reinterpret_cast<T *>(smem_raw);  // [BS][BS+1]
   T *X = M + BS * (BS + 1);                // [BS][BS+1]
-  constexpr int LD = BS + 1;
-  const int b = blockIdx.x, j = threadIdx.x;
+  constexpr int LD = BS + 1, NT = 4 * BS, NL = BS * BS / NT;
+  const int b = blockIdx.x, t = threadIdx.x, j = t >> 2, h = t & 3;
   const bool upper = blockIdx.y == 1;
   const int r0 = b * BS;
   const int nb = n - r0 < BS ? n - r0 : BS;
-  for (int e = j; e < BS * BS; e += BS) {
-    const int r = e / BS, c = e % BS;
-    M[r * LD + c] = (r < nb && c < nb) ? lu[(int64_t)(r0 + r) * lda + r0 + c] : T(0);
-    X[r * LD + c] = T(0);
+  {
+    T v[NL];
+#pragma unroll
+    for (int q = 0; q < NL; ++q) {
+      const int e = t + q * NT, r = e / BS, c = e % BS;
+      v[q] = (r < nb && c < nb) ? lu[(int64_t)(r0 + r) * lda + r0 + c] : T(0);
+    }
+#pragma unroll
+    for (int q = 0; q < NL; ++q) {
+      const int e = t + q * NT, r = e / BS, c = e % BS;
+      M[r * LD + c] = v[q];
+      X[r * LD + c] = T(0);
+    }
   }
   __syncthreads();
-  // Column j of the inverse by substitution; each entry's dot product runs
-  // over four accumulators, eight terms per step with their LDS loads issued
-  // together (the loads, not the multiply-adds, set the time).
-  auto dot = [&](int i, int p0, int p1) -> T {  // sum over p in [p0, p1) of M[i][p] X[p][j]
-    T a[4] = {T(0), T(0), T(0), T(0)};
-    int p = p0;
-    for (; p + 8 <= p1; p += 8) {
-      T m[8], x[8];
+  // Sum over p in [p0, p1) of M[i][p] X[p][j].
+  auto dot = [&](int i, int p0, int p1) -> T {
+    T a = T(0);
+    for (int p = p0 + h; p < p1; p += 16) {
+      T m[4], x[4];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        m[q] = M[i * LD + p + q];
-        x[q] = X[(p + q) * LD + j];
+      for (int q = 0; q < 4; ++q) {
+        const int k = p + 4 * q, kc = k < p1 ? k : p;
+        m[q] = M[i * LD + kc];
+        x[q] = X[kc * LD + j];
       }
 #pragma unroll
-      for (int q = 0; q < 8; ++q) a[q & 3] += m[q] * x[q];
+      for (int q = 0; q < 4; ++q)
+        if (p + 4 * q < p1) a += m[q] * x[q];
     }
-    for (; p < p1; ++p) a[p & 3] += M[i * LD + p] * X[p * LD + j];
-    return (a[0] + a[1]) + (a[2] + a[3]);
+    a += quad_xor<0xB1>(a);  // lanes 1, 0, 3, 2
+    a += quad_xor<0x4E>(a);  // lanes 2, 3, 0, 1
+    return a;
   };
+  // Column j of the inverse by substitution (its four lanes are in one wave).
   if (j < nb) {
     if (!upper) {
-      X[j * LD + j] = T(1);
-      for (int i = j + 1; i < nb; ++i) X[i * LD + j] = -dot(i, j, i);
+      if (h == 0) X[j * LD + j] = T(1);
+      for (int i = j + 1; i < nb; ++i) {
+        __asm__ volatile("" ::: "memory");  // the quad's store comes before its loads
+        const T d = dot(i, j, i);
+        if (h == 0) X[i * LD + j] = -d;
+      }
     } else {
-      X[j * LD + j] = T(1) / M[j * LD + j];
-      for (int i = j - 1; i >= 0; --i) X[i * LD + j] = -dot(i, i + 1, j + 1) / M[i * LD + i];
+      if (h == 0) X[j * LD + j] = T(1) / M[j * LD + j];
+      for (int i = j - 1; i >= 0; --i) {
+        __asm__ volatile("" ::: "memory");  // the quad's store comes before its loads
+        const T d = -dot(i, i + 1, j + 1) / M[i * LD + i];
+        if (h == 0) X[i * LD + j] = d;
+      }
     }
   }
   __syncthreads();
   T *out = (upper ? uinv : linv) + (size_t)b * BS * BS;
-  for (int e = j; e < BS * BS; e += BS) out[e] = X[(e / BS) * LD + e % BS];
+  for (int e = t; e < BS * BS; e += NT) out[e] = X[(e / BS) * LD + e % BS];
 }
 
 template <typename T>
@@ -676,7 +708,7 @@ hipError_t launch_trtri_diag(lair_context *ctx, const T *lu, int64_t lda, int n,
   static bool once = (allow_large_lds(trtri_diag_kernel<T, BS>), true);
   (void)once;
   const int slot = prof_begin(ctx, LAIR_KCLASS_GETRS);
-  trtri_diag_kernel<T, BS><<<dim3(nblk, 2), BS, shm, ctx->stream>>>(lu, lda, n, linv, uinv);
+  trtri_diag_kernel<T, BS><<<dim3(nblk, 2), 4 * BS, shm, ctx->stream>>>(lu, lda, n, linv, uinv);
   prof_end(ctx, slot, LAIR_KCLASS_GETRS, (double)nblk * BS * BS * BS / 3.0);
   return hipGetLastError();
 }
