@@ -206,6 +206,7 @@ __global__ void __launch_bounds__(256, 2) cgetrs_flow_kernel(CflowArgs<T> p) {
   const int gr = min(r0 + r, p.n - 1);
   unsigned long long *xt = p.xt + (int64_t)c * p.n * WPE;
   if (t < 2) s_bail[t] = 0;
+  __syncthreads();  // before a wave's first wait may set a flag
 
   for (int e = t; e < BS * BS; e += 256) {
     const int row = e / BS, k = e % BS;

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 import lair_amd as L
-from lair_amd import inputs
+from lair_amd import _capi, inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -34,3 +34,30 @@ def test_complex_getrs_blocks(n, nrhs, scale, dtype):
     r = b.astype(np.complex128) - a128 @ x
     berr = np.abs(r).max(0) / (np.abs(a128).sum(1).max() * np.abs(x).max(0))
     assert berr.max() <= 8 * n * float(np.finfo(dtype).eps)
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("n,nrhs", [(129, 1), (300, 3)])
+def test_complex_getrs_waits_give_up(n, nrhs, dtype):
+    """A wait limit of 0 ends the first wait of every workgroup at once: the
+    call reports it, and the next call on the context solves."""
+    a = (inputs.gaussian_matrix(8300 + n, n, n) + 4.0 * np.sqrt(n) * np.eye(n)).astype(dtype)
+    b = inputs.gaussian_matrix(8400 + n, n, nrhs).astype(dtype)
+    g = a.copy()
+    piv, _ = L.getrf(g)
+    ctx = L.Context()
+    fn = ctx.lib.lair_zgetrs_device if dtype == np.complex128 else ctx.lib.lair_cgetrs_device
+    dlu, dp, db = L.DeviceArray.from_host(g), L.DeviceArray.from_host(piv.reshape(-1, 1)), L.DeviceArray.from_host(b)
+    args = (ctx.h, n, nrhs, dlu.ptr, n, dp.ptr, db.ptr, nrhs)
+    L.check(ctx.lib.lair_context_set_wait_limit(ctx.h, 0), "wait limit")
+    try:
+        st = fn(*args)
+    finally:
+        L.check(ctx.lib.lair_context_set_wait_limit(ctx.h, 1 << 23), "wait limit")
+    assert st == _capi.LAIR_ERR_SYNC
+    db.upload(b)
+    L.check(fn(*args), "getrs")
+    np.testing.assert_array_equal(db.download(), L.getrs(g, piv, b))
+    for d in (dlu, dp, db):
+        d.free()
+    ctx.close()
