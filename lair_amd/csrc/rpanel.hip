@@ -407,6 +407,7 @@ __global__ void __launch_bounds__(kRpThreads) rpanel_kernel(RpArgs<T> pa) {
     const int cw = min(W, ncols - c0);    // columns of the sub-panel
     const int np = min(W, pa.npiv - c0);  // pivots of the sub-panel
     uint32_t now[RPT];                    // rows that became pivot rows in this sub-panel
+    unsigned skip = 0;                    // its columns without a candidate
     T v[RPT][W];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
@@ -593,10 +594,12 @@ __global__ void __launch_bounds__(kRpThreads) rpanel_kernel(RpArgs<T> pa) {
           }
         }
       } else {
-        // A column without a nonzero candidate is left unscaled
-        // (getrf.rs:72-73); the row at position d is the pivot row.
+        // A column without a nonzero candidate is left unscaled and nothing
+        // is eliminated with it (getrf.rs:72-73); the row at position d is the
+        // pivot row.
         pw = d;
         last_none = d;
+        skip |= 1u << j;
 #pragma unroll
         for (int s = 0; s < RPT; ++s) {
           s_l[j * LP + r0 + 64 * s] = v[s][0];
@@ -757,7 +760,21 @@ __global__ void __launch_bounds__(kRpThreads) rpanel_kernel(RpArgs<T> pa) {
     }
     if (rest <= 0) break;
     // U = L11^-1 A, one thread per column.
-    if (t < rest) {
+    skip = (unsigned)__builtin_amdgcn_readfirstlane((int)skip);
+    if (__builtin_expect(skip != 0, 0)) {
+      if (t < rest)
+#pragma unroll 1
+        for (int i = 1; i < np; ++i) {
+          T x = s_u[i * un + t];
+#pragma unroll 1
+          for (int q = 0; q < i; ++q)
+            if (!(skip >> q & 1u)) {
+              const T e = s_lt[i * W + q] * s_u[q * un + t];
+              x = x - e;
+            }
+          s_u[i * un + t] = x;
+        }
+    } else if (t < rest) {
       T x[W];
 #pragma unroll
       for (int i = 0; i < W; ++i) x[i] = s_u[i * un + t];
@@ -789,6 +806,20 @@ __global__ void __launch_bounds__(kRpThreads) rpanel_kernel(RpArgs<T> pa) {
         for (int e = 0; e < 2; ++e)
           if (lane_o + 64 * e < rest) dst[lane_o + 64 * e] = s_u[j * un + lane_o + 64 * e];
       }
+    }
+    if (__builtin_expect(skip != 0, 0)) {
+      // The update passes over columns without a candidate: with zeros for the
+      // column of L and the row of U, both stored by now, it subtracts 0 from
+      // every entry (their own values may be NaN, or meet an infinity).
+      __syncthreads();
+#pragma unroll 1
+      for (int j = 0; j < np; ++j)
+        if (skip >> j & 1u) {
+#pragma unroll
+          for (int s = 0; s < RPT; ++s) s_lc[j * LP + r0 + 64 * s] = T(0);
+          if (t < un) s_u[j * un + t] = T(0);
+        }
+      __syncthreads();
     }
     // A22 -= L21 U on this wave's rows.  The next sub-panel's columns come
     // last and stay in LDS; with kDefer the whole blocks beyond them wait.

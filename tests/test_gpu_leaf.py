@@ -74,3 +74,19 @@ def test_leaf_extreme_values(m, dt):
     a[7, 4] = np.nan
     a[m - 1, 9] = np.inf
     _same_as_oracle(a, 20)
+
+
+@pytest.mark.parametrize("dt", TYPES)
+@pytest.mark.parametrize("m", [300, 700, 1500, 2500, 17000])
+@pytest.mark.parametrize("value", [0.0, np.nan])
+def test_leaf_skips_columns_without_candidate(m, value, dt):
+    """Nothing is eliminated with a column of zeros or NaN, neither in its own
+    sub-panel nor right of it: an infinity in its pivot row (the diagonal is
+    dominant, so row c is at position c) stays the only one of its column, and
+    the NaN stay in theirs."""
+    a = _gauss(1200 + m, m, 64, dt)
+    a[np.arange(64), np.arange(64)] += 100
+    for c in (0, 5, 18):
+        a[:, c] = value
+        a[c, c + 20] = np.inf
+    _same_as_oracle(a, 64)
