@@ -8,6 +8,8 @@ A matrix of at most 64 columns is one leaf, whose operations are those of
 getrf_row_major (src/lapack/getrf.rs:55-117) in the same order, so pivots and
 factors have to equal the oracle's bit for bit; no tolerance is involved.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -90,3 +92,34 @@ def test_leaf_skips_columns_without_candidate(m, value, dt):
         a[:, c] = value
         a[c, c + 20] = np.inf
     _same_as_oracle(a, 64)
+
+
+@pytest.mark.parametrize("dt", TYPES)
+@pytest.mark.parametrize("shape", [(2049, 64), (4097, 64), (8193, 64), (16385, 64), (33000, 48)])
+def test_leaf_whole_blocks_beyond_sub_panels(shape, dt):
+    """Whole blocks of columns right of the next sub-panel, whose update is put
+    off (up to 16384 rows) or not, with every number of records a wave polls;
+    33000 rows: more than 32 workgroups."""
+    m, n = shape
+    if dt == np.complex128 and m > 32768:
+        pytest.skip("zgetrf takes at most 32768 rows")
+    _same_as_oracle(_gauss(500 + m + n, m, n, dt), n)
+
+
+@pytest.mark.parametrize("m", [512, 1300, 9000, 17000])
+def test_leaf_of_128_fp32_columns(m):
+    """The widest leaf: eight sub-panels in one launch."""
+    a = _gauss(700 + m, m, 128, np.float32)
+    ref = a.copy()
+    piv_o, sing_o = O.sgetrf(ref)
+    ctx = L.Context()
+    da, dp = L.DeviceArray.from_host(a), L.DeviceArray(128, 1, np.int64)
+    sing = ctypes.c_int64(-1)
+    L.check(ctx.lib.lair_sgetrf_device(ctx.h, m, 128, da.ptr, 128, dp.ptr, 128, ctypes.byref(sing)), "getrf")
+    piv, lu = dp.download().ravel(), da.download()
+    da.free()
+    dp.free()
+    ctx.close()
+    assert sing_o is None and sing.value == -1
+    assert np.array_equal(piv, piv_o)
+    assert np.array_equal(lu, ref)
