@@ -214,6 +214,9 @@ static lair_status getrf_impl(lair_context *ctx, int64_t m64, int64_t n64, T *a,
   auto leaf_width = [&](int k, int kb) -> int {
     return tournament ? 0 : rpanel_leaf_width<T>(ctx, kb, m - k);
   };
+  // Columns of the update that runs beside the panel at column k (the first
+  // panel runs alone).
+  auto beside = [&](int k, int kb) -> int { return k > 0 ? n - (k + kb) : 0; };
   // Factors the panel of columns [k, k + kb) on the context's stream.
   auto factor_panel = [&](int k, int kb) -> hipError_t {
     // Resident leaves.  A leaf narrower than the panel is followed by its
@@ -225,9 +228,9 @@ static lair_status getrf_impl(lair_context *ctx, int64_t m64, int64_t n64, T *a,
     if (lw > 0) {
       for (int c = k; c < k + kb; c += lw) {
         const int w = std::min(lw, k + kb - c);
-        hipError_t e2 = pmap_ok[pp] ? launch_rpanel<T>(ctx, a, lda, c, m, c, w, ipiv, ctx->pmap_rows[pp],
-                                                       ctx->pmap_src[pp], ctx->pmap_count[pp])
-                                    : launch_rpanel<T>(ctx, a, lda, c, m, c, w, ipiv);
+        hipError_t e2 = pmap_ok[pp] ? launch_rpanel<T>(ctx, a, lda, c, m, c, w, beside(k, kb), ipiv,
+                                                       ctx->pmap_rows[pp], ctx->pmap_src[pp], ctx->pmap_count[pp])
+                                    : launch_rpanel<T>(ctx, a, lda, c, m, c, w, beside(k, kb), ipiv);
         if (e2 != hipSuccess) return e2;
         const int npv = std::min(w, m - c);
         if (npv <= 0) continue;
@@ -317,7 +320,7 @@ static lair_status getrf_impl(lair_context *ctx, int64_t m64, int64_t n64, T *a,
   auto reserve_for = [&](int k) {
     const int kb = std::min<int>((int)nb, kmax - k);
     const int lw = k < kmax ? leaf_width(k, kb) : 0;
-    ctx->panel_wgs = lw > 0 ? rpanel_grid<T>(ctx, m - k) : 0;
+    ctx->panel_wgs = lw > 0 ? rpanel_grid<T>(ctx, m - k, beside(k, kb)) : 0;
   };
   // Look-ahead of depth one.  Stream 1 (the context's stream) carries the
   // critical path: panel k+1's columns are updated first, then panel k+1 is

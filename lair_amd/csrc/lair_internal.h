@@ -222,10 +222,12 @@ hipError_t launch_panel(lair_context *ctx, T *a, int64_t lda, int row0, int m, i
                         int64_t *ipiv, int rest1, int left0);
 // Resident-panel leaf (rpanel.hip): exact partial pivoting of columns
 // [col0, col0 + wcols) over rows [row0, m), wcols at most the leaf width.
+// beside: columns of the trailing update that runs at the same time (the
+// leaf's workgroups and those of the update share the CUs).
 // When map_rows is given, the leaf also writes the row map of its
 // interchanges (2 * npiv gather entries, see launch_rowswap_map).
 template <typename T>
-hipError_t launch_rpanel(lair_context *ctx, T *a, int64_t lda, int row0, int m, int col0, int wcols,
+hipError_t launch_rpanel(lair_context *ctx, T *a, int64_t lda, int row0, int m, int col0, int wcols, int beside,
                          int64_t *ipiv, int *map_rows = nullptr, int *map_src = nullptr,
                          int *map_count = nullptr);
 // Widest leaf <= want the resident panel supports for `rows` rows, or 0.
@@ -233,7 +235,7 @@ template <typename T>
 int rpanel_leaf_width(lair_context *ctx, int want, int rows);
 // Workgroups of a resident leaf over `rows` rows (0: unsupported).
 template <typename T>
-int rpanel_grid(lair_context *ctx, int rows);
+int rpanel_grid(lair_context *ctx, int rows, int beside);
 // Tournament-pivoting FP32 leaf (mixed-precision factorization only).
 hipError_t launch_panel_calu(lair_context *ctx, float *a, int64_t lda, int c, int m, int wcols,
                              int64_t *ipiv, int rest1, int left0);

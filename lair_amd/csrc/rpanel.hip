@@ -52,25 +52,13 @@
 
 namespace lair {
 
-// Sub-panel width: its record (W entries, a reciprocal and the position) is
-// one 64-bit word per lane.
+// Sub-panel width: its record (W entries, the position and the row) is one
+// 64-bit word per lane.  Complex rows cost four times the arithmetic, and half
+// of a sub-panel's entries are retired on average, so they take 8: complex<f32>
+// 64 columns of 3000 rows 318 us against 327 with 16.
 template <typename T>
-struct RpW;
-template <>
-struct RpW<float> {
-  static constexpr int W = 16;
-};
-template <>
-struct RpW<double> {
-  static constexpr int W = 16;
-};
-template <>
-struct RpW<ccplx> {
-  static constexpr int W = 16;
-};
-template <>
-struct RpW<zcplx> {
-  static constexpr int W = 8;
+struct RpW {
+  static constexpr int W = cplx_traits<T>::is ? 8 : 16;
 };
 
 template <typename T>
@@ -1026,38 +1014,75 @@ static hipError_t rp_launch(lair_context *ctx, const RpArgs<T> &pa) {
   return hipGetLastError();
 }
 
-// Rows per thread of a leaf over `rows` rows, or 0 when the leaf does not fit
-// the cooperating workgroups.
+// Several workgroups, one or two rows per thread: the fewest records a wave
+// has to poll.  (Complex leaves of two rows per thread have more than 32
+// workgroups, unless the workgroups are capped.)
 template <typename T>
-static int rp_rpt(lair_context *ctx, int rows) {
+static hipError_t rp_launch_multi(lair_context *ctx, const RpArgs<T> &pa, int rpt) {
+  if constexpr (cplx_traits<T>::is) {
+    if (rpt == 2) return rp_launch<T, 2, 16>(ctx, pa);
+  }
+  constexpr int RPT = cplx_traits<T>::is ? 1 : 2;
+  const int mr = (pa.P + kRpWaves - 1) / kRpWaves;
+  if (mr <= 1) return rp_launch<T, RPT, 1>(ctx, pa);
+  if (mr <= 2) return rp_launch<T, RPT, 2>(ctx, pa);
+  if (mr <= 4) return rp_launch<T, RPT, 4>(ctx, pa);
+  if (mr <= 8) return rp_launch<T, RPT, 8>(ctx, pa);
+  return rp_launch<T, RPT, 16>(ctx, pa);
+}
+
+// Rows per thread of a leaf over `rows` rows, or 0 when the leaf does not fit
+// the cooperating workgroups.  `beside`: columns of the trailing update that
+// runs at the same time.
+//
+// More rows per thread save exchanges (one workgroup needs none), fewer save
+// arithmetic per column.  A factorization of m x 64, call included, us:
+//   rows        f64: 4 a thread, one workgroup / 2, two workgroups  226 / 262
+//   513 - 1024  f32                                                 206 / 243
+//               complex: 4, one / 2, two / 1, four  f32: 336 / 302 / 262
+//                                                   f64: 418 / 338 / 294
+//   3000        complex: 2, six / 1, twelve         f32: 325 / 264, f64: 354 / 300
+//   20000       4, twenty / 2, forty   f64: 374 / 299, f32: 349 / 288,
+//                                      complex f32: 491 / 347, f64: 588 / 405
+// Beyond 32 workgroups the trailing update loses as many CUs, so there the
+// leaf has 4 rows a thread while that update sets the pace.  The two cross at
+// about 24000 bytes of a row beside the panel: 24000 rows of n columns gain
+// most at n = 6000 in f32 (34.3 against 25.9 ms), 3000 in f64 (17.9 / 15.3) and
+// complex<f32> (23.4 / 19.2), 1500 - 2000 in complex<f64> (19.9 / 16.2), and
+// lose beyond n = 14000 in f32 (78.8 / 81).
+constexpr int64_t kRpBesideBytes = 24000;
+template <typename T>
+static int rp_rpt(lair_context *ctx, int rows, int beside) {
   const int maxp = std::min(ctx->rp_max_wg, kMaxPanelWG);
   // Complex<f64> keeps to 32768 rows, the limit its entry points state.
   if (sizeof(T) == 16 && rows > 32768) return 0;
   if (rows <= kRpThreads) return 1;
   if (rows <= 2 * kRpThreads) return 2;
+  if (cplx_traits<T>::is && rows <= kRpThreads * maxp) return 1;
   if (rows <= 4 * kRpThreads) return 4;
   if (rows <= 2 * kRpThreads * std::min(maxp, 32)) return 2;
+  if (rows <= 2 * kRpThreads * maxp && beside * (int64_t)sizeof(T) <= kRpBesideBytes) return 2;
   return rows <= 4 * kRpThreads * maxp ? 4 : 0;
 }
 
 template <typename T>
-int rpanel_grid(lair_context *ctx, int rows) {
-  const int nr = rp_rpt<T>(ctx, rows) * kRpThreads;
+int rpanel_grid(lair_context *ctx, int rows, int beside) {
+  const int nr = rp_rpt<T>(ctx, rows, beside) * kRpThreads;
   return nr > 0 ? (rows + nr - 1) / nr : 0;
 }
 
 // Widest leaf (<= want) for `rows` rows.
 template <typename T>
 int rpanel_leaf_width(lair_context *ctx, int want, int rows) {
-  return rpanel_grid<T>(ctx, rows) > 0 ? std::min(want, RpLds<T, 1, 0>::NBM) : 0;
+  return rpanel_grid<T>(ctx, rows, 0) > 0 ? std::min(want, RpLds<T, 1, 0>::NBM) : 0;
 }
 
 template <typename T>
-hipError_t launch_rpanel(lair_context *ctx, T *a, int64_t lda, int row0, int m, int col0, int wcols,
+hipError_t launch_rpanel(lair_context *ctx, T *a, int64_t lda, int row0, int m, int col0, int wcols, int beside,
                          int64_t *ipiv, int *map_rows, int *map_src, int *map_count) {
   const int rows = m - row0;
   if (rows <= 0 || wcols <= 0) return hipSuccess;
-  const int rpt = rp_rpt<T>(ctx, rows);
+  const int rpt = rp_rpt<T>(ctx, rows, beside);
   if (rpt == 0 || wcols > RpLds<T, 1, 0>::NBM) return hipErrorInvalidValue;
   // A reused tag could match a stale word: clear the buffers and restart the
   // tags before they wrap.
@@ -1074,7 +1099,7 @@ hipError_t launch_rpanel(lair_context *ctx, T *a, int64_t lda, int row0, int m, 
   pa.col0 = col0;
   pa.wcols = wcols;
   pa.npiv = wcols < rows ? wcols : rows;
-  pa.P = rpanel_grid<T>(ctx, rows);
+  pa.P = rpanel_grid<T>(ctx, rows, beside);
   pa.ipiv = ipiv;
   pa.sing = ctx->sing;
   pa.map_rows = map_rows;
@@ -1092,10 +1117,8 @@ hipError_t launch_rpanel(lair_context *ctx, T *a, int64_t lda, int row0, int m, 
     e = rpt == 1 ? rp_launch<T, 1, 0>(ctx, pa) : (rpt == 2 ? rp_launch<T, 2, 0>(ctx, pa) : rp_launch<T, 4, 0>(ctx, pa));
   else if (rpt == 4)
     e = rp_launch<T, 4, 16>(ctx, pa);
-  else if (pa.P <= 8)
-    e = pa.P <= 4 ? rp_launch<T, 2, 1>(ctx, pa) : rp_launch<T, 2, 2>(ctx, pa);
   else
-    e = pa.P <= 16 ? rp_launch<T, 2, 4>(ctx, pa) : rp_launch<T, 2, 8>(ctx, pa);
+    e = rp_launch_multi<T>(ctx, pa, rpt);
   prof_end(ctx, slot, LAIR_KCLASS_PANEL, (double)pa.npiv * rows * wcols,
            2.0 * sizeof(T) * (double)rows * wcols);
   ctx->rp_seq += kRpTags;
@@ -1103,9 +1126,10 @@ hipError_t launch_rpanel(lair_context *ctx, T *a, int64_t lda, int row0, int m, 
 }
 
 #define LAIR_RP_INST(T)                                                                                \
-  template int rpanel_grid<T>(lair_context *, int);                                                    \
+  template int rpanel_grid<T>(lair_context *, int, int);                                               \
   template int rpanel_leaf_width<T>(lair_context *, int, int);                                         \
-  template hipError_t launch_rpanel<T>(lair_context *, T *, int64_t, int, int, int, int, int64_t *, int *, int *, int *);
+  template hipError_t launch_rpanel<T>(lair_context *, T *, int64_t, int, int, int, int, int, int64_t *, int *,        \
+                                       int *, int *);
 LAIR_RP_INST(float)
 LAIR_RP_INST(double)
 LAIR_RP_INST(zcplx)

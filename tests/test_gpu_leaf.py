@@ -1,8 +1,9 @@
 """The panel leaf (rpanel.hip) at the sizes where its plan changes: one
 workgroup with 1, 2 or 4 rows per thread (256, 512, 1024 rows), several
-workgroups (from 1025 rows, by the number of records a wave polls: 2048, 4096,
-8192 rows; from 16385 with 4 rows per thread), sub-panels of 16 (complex<f64>:
-8) columns and ragged last ones.
+workgroups (real types from 1025 rows with 2 rows per thread, complex ones from
+513 with 1, by the number of records a wave polls; beyond 32 workgroups of 2
+rows per thread with 2 or 4), sub-panels of 16 (complex: 8) columns and ragged
+last ones.
 
 A matrix of at most 64 columns is one leaf, whose operations are those of
 getrf_row_major (src/lapack/getrf.rs:55-117) in the same order, so pivots and
@@ -123,3 +124,38 @@ def test_leaf_of_128_fp32_columns(m):
     assert sing_o is None and sing.value == -1
     assert np.array_equal(piv, piv_o)
     assert np.array_equal(lu, ref)
+
+
+@pytest.mark.parametrize("dt", TYPES)
+@pytest.mark.parametrize("shape", [(513, 64), (769, 40), (1025, 9), (4096, 24), (8192, 33), (16384, 17), (32768, 40)])
+def test_leaf_plan_edges(shape, dt):
+    """The last sizes of a plan and the first of the next."""
+    m, n = shape
+    _same_as_oracle(_gauss(800 + m + n, m, n, dt), n)
+
+
+@pytest.mark.parametrize("dt,m,n", [(np.float64, 17000, 3200), (np.float32, 17000, 200), (np.complex128, 17000, 200),
+                                    (np.complex64, 17000, 200), (np.complex64, 3000, 300)])
+def test_leaf_factors_do_not_depend_on_the_plan(dt, m, n, monkeypatch):
+    """At most 8, 32 and 64 workgroups: 1, 2 or 4 rows per thread for the same
+    rows (f64: wide enough for the trailing update to decide as well).  Each
+    leaf does the same operations, so the factors are the same bits."""
+    rng = np.random.default_rng(m + n)
+    a = rng.standard_normal((m, n))
+    a = (a + 1j * rng.standard_normal((m, n)) if np.dtype(dt).kind == "c" else a).astype(dt)
+    name = {np.float64: "d", np.float32: "s", np.complex128: "z", np.complex64: "c"}[dt]
+    out = []
+    for wgs in (8, 32, 64) if m <= 8192 else (32, 64):
+        monkeypatch.setenv("LAIR_PANEL_MAX_WG", str(wgs))
+        ctx = L.Context()
+        da, dp = L.DeviceArray.from_host(a), L.DeviceArray(n, 1, np.int64)
+        sing = ctypes.c_int64(-1)
+        L.check(getattr(ctx.lib, f"lair_{name}getrf_device")(ctx.h, m, n, da.ptr, n, dp.ptr, 0, ctypes.byref(sing)),
+                "getrf")
+        out.append((dp.download(), da.download()))
+        da.free()
+        dp.free()
+        ctx.close()
+    for piv, lu in out[1:]:
+        assert np.array_equal(piv, out[0][0])
+        assert np.array_equal(lu, out[0][1])
