@@ -260,6 +260,7 @@ __global__ void __launch_bounds__(kRpThreads) rpanel_kernel(RpArgs<T> pa) {
   __shared__ int s_po[kRpMaxCols];  // rows that the pivot rows were loaded from
   __shared__ __align__(16) int s_pw[kRpMaxCols];  // pivot positions of the leaf
   __shared__ int s_cnt, s_bail;
+  __shared__ unsigned s_skip;  // columns of the sub-panel without a candidate
 
   const int g = blockIdx.x, t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -283,6 +284,7 @@ __global__ void __launch_bounds__(kRpThreads) rpanel_kernel(RpArgs<T> pa) {
   if (t == 0) {
     s_bail = pa.wait_limit <= 0 ? 1 : 0;
     s_cnt = 0;
+    s_skip = 0;
   }
   __syncthreads();
   bool bail = s_bail != 0;
@@ -395,7 +397,6 @@ __global__ void __launch_bounds__(kRpThreads) rpanel_kernel(RpArgs<T> pa) {
     const int cw = min(W, ncols - c0);    // columns of the sub-panel
     const int np = min(W, pa.npiv - c0);  // pivots of the sub-panel
     uint32_t now[RPT];                    // rows that became pivot rows in this sub-panel
-    unsigned skip = 0;                    // its columns without a candidate
     T v[RPT][W];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
@@ -587,7 +588,7 @@ __global__ void __launch_bounds__(kRpThreads) rpanel_kernel(RpArgs<T> pa) {
         // pivot row.
         pw = d;
         last_none = d;
-        skip |= 1u << j;
+        if (t == 0) s_skip |= 1u << j;
 #pragma unroll
         for (int s = 0; s < RPT; ++s) {
           s_l[j * LP + r0 + 64 * s] = v[s][0];
@@ -748,7 +749,7 @@ __global__ void __launch_bounds__(kRpThreads) rpanel_kernel(RpArgs<T> pa) {
     }
     if (rest <= 0) break;
     // U = L11^-1 A, one thread per column.
-    skip = (unsigned)__builtin_amdgcn_readfirstlane((int)skip);
+    const unsigned skip = (unsigned)__builtin_amdgcn_readfirstlane((int)s_skip);
     if (__builtin_expect(skip != 0, 0)) {
       if (t < rest)
 #pragma unroll 1
@@ -784,6 +785,7 @@ __global__ void __launch_bounds__(kRpThreads) rpanel_kernel(RpArgs<T> pa) {
         if (i < np) s_u[i * un + t] = x[i];
     }
     __syncthreads();
+    if (t == 0) s_skip = 0;
     // The pivot rows' entries right of the sub-panel, by their owners.
 #pragma unroll
     for (int i = 0; i < JW; ++i) {
