@@ -484,14 +484,15 @@ template bool gemm_small_fits<double>(const lair_context *, int, int, int64_t, i
 template bool gemm_small_fits<float>(const lair_context *, int, int, int64_t, int64_t, int64_t);
 
 // Splits C into the region of whole tiles (unmasked kernel, launched by
-// `interior`) and the right and bottom strips (launched by `masked`: small
-// tiles where there is such a kernel, else the masked one; 4000 x 2000 x 128 in
-// FP64 with its strips: 86 against 128 us); K not a multiple of the stage depth
-// runs so throughout.  The 32-bit buffer offsets need 128 rows of C, A and B
-// within 2 GiB.
-template <typename T, bool TRANSA, typename FI, typename FM>
+// `interior`) and the right and bottom strips (launched by `strip`: small tiles
+// where there is such a kernel, else the masked one; 4000 x 2000 x 128 in FP64
+// with its strips: 86 against 128 us).  K not a multiple of the stage depth runs
+// masked throughout (`masked`), on large tiles: FP64 4096 x 4096 x 100 129 us
+// against 175 with small ones, 2048 x 2048 x 1000 234 / 312, FP32 88 / 111 and
+// 163 / 274.  The 32-bit buffer offsets need 128 rows of C, A and B within 2 GiB.
+template <typename T, bool TRANSA, typename FI, typename FS, typename FM>
 static hipError_t split_tiles(int M, int N, int K, int kstep, const T *A, int64_t lda, const T *B, int64_t ldb,
-                              T *C, int64_t ldc, FI interior, FM masked) {
+                              T *C, int64_t ldc, FI interior, FS strip, FM masked) {
   const int64_t big = std::max(std::max(lda, ldb), ldc);
   if (big > ((int64_t)1 << 31) / ((int64_t)kTileM * (int64_t)sizeof(T))) return hipErrorInvalidValue;
   if (K % kstep != 0) {
@@ -501,25 +502,29 @@ static hipError_t split_tiles(int M, int N, int K, int kstep, const T *A, int64_
   const int Mf = M / kTileM * kTileM, Nf = N / kTileN * kTileN;
   if (Mf > 0 && Nf > 0) interior(Mf, Nf);
   // Right strip (rows of the interior), then the bottom strip (all columns).
-  masked(Mf, N - Nf, A, B + Nf, C + Nf);
-  masked(M - Mf, N, TRANSA ? A + Mf : A + (int64_t)Mf * lda, B, C + (int64_t)Mf * ldc);
+  strip(Mf, N - Nf, A, B + Nf, C + Nf);
+  strip(M - Mf, N, TRANSA ? A + Mf : A + (int64_t)Mf * lda, B, C + (int64_t)Mf * ldc);
   return hipGetLastError();
 }
 
 template <typename T, bool TRANSA, bool STORE, typename F>
 static hipError_t gemm_split(lair_context *ctx, int M, int N, int K, const T *A, int64_t lda, const T *B,
                              int64_t ldb, T *C, int64_t ldc, F interior) {
-  [[maybe_unused]] hipStream_t st = ctx->stream;
   auto masked = [&](int m, int n, const T *a, const T *b, T *c) {
     if (m <= 0 || n <= 0) return;
-    if constexpr (!TRANSA && !STORE) {
-      (void)launch_gemm_small<T>(ctx, m, n, K, a, lda, b, ldb, c, ldc);
-    } else {
-      const unsigned g = (unsigned)(((m + kTileM - 1) / kTileM) * ((n + kTileN - 1) / kTileN));
-      gemm_tile_kernel<T, TRANSA, STORE, 1, true><<<g, 256, 0, st>>>(m, n, K, a, lda, b, ldb, c, ldc);
-    }
+    const unsigned g = (unsigned)(((m + kTileM - 1) / kTileM) * ((n + kTileN - 1) / kTileN));
+    gemm_tile_kernel<T, TRANSA, STORE, 1, true><<<g, 256, 0, ctx->stream>>>(m, n, K, a, lda, b, ldb, c, ldc);
   };
-  return split_tiles<T, TRANSA>(M, N, K, kBK, A, lda, B, ldb, C, ldc, interior, masked);
+  if constexpr (!TRANSA && !STORE) {
+    hipError_t se = hipSuccess;
+    auto strip = [&](int m, int n, const T *a, const T *b, T *c) {
+      if (m > 0 && n > 0 && se == hipSuccess) se = launch_gemm_small<T>(ctx, m, n, K, a, lda, b, ldb, c, ldc);
+    };
+    const hipError_t e = split_tiles<T, TRANSA>(M, N, K, kBK, A, lda, B, ldb, C, ldc, interior, strip, masked);
+    return e != hipSuccess ? e : se;
+  } else {
+    return split_tiles<T, TRANSA>(M, N, K, kBK, A, lda, B, ldb, C, ldc, interior, masked, masked);
+  }
 }
 
 hipError_t launch_dgemm_tile(lair_context *ctx, int M, int N, int K, const double *A, int64_t lda,
@@ -783,7 +788,7 @@ hipError_t launch_bgemm_tile(lair_context *ctx, int ns, int M, int N, int K, con
         bgemm_tile_kernel<NS, 1, false><<<(unsigned)(nbm * nbn), 256, 0, st>>>(m, n, K, A, lda, B, ldb, C, ldc);
       }
     };
-    return split_tiles<float, false>(M, N, K, kBBK, A, lda, B, ldb, C, ldc, interior, masked);
+    return split_tiles<float, false>(M, N, K, kBBK, A, lda, B, ldb, C, ldc, interior, masked, masked);
   };
   return ns == 3 ? run(std::integral_constant<int, 3>{}) : run(std::integral_constant<int, 1>{});
 }
