@@ -671,11 +671,73 @@ __global__ void __launch_bounds__(64 * kExactWaves)
   if (i1 < n) b[(int64_t)i1 * ldb + c] = x1;
 }
 
+// Many right-hand sides: one thread per right-hand side, x in LDS, the same
+// operations in the same order.  Bound by each thread's chain of loads of the
+// factors, whatever the number of right-hand sides that the chip holds at once.
+template <typename T>
+__global__ void __launch_bounds__(64)
+    getrs_exact_many_kernel(int n, int nrhs, const T *lu, int64_t lda, const int64_t *ipiv, T *b, int64_t ldb,
+                            int32_t *status) {
+#pragma clang fp contract(off)
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  T *xs = reinterpret_cast<T *>(smem_raw);  // [n][64]
+  const int t = threadIdx.x;
+  const int c = blockIdx.x * 64 + t;
+  if (c >= nrhs) return;
+  for (int i = 0; i < n; ++i) xs[i * 64 + t] = b[(int64_t)i * ldb + c];
+  for (int i = 0; i < n; ++i) {
+    const int64_t p64 = ipiv[i];
+    if (p64 < 0 || p64 >= n) {  // outside [0, n): skipped and reported
+      if (t == 0) atomic_or_agent(status, kErrPivot);
+      continue;
+    }
+    const int p = (int)p64;
+    if (p != i) {
+      const T tmp = xs[i * 64 + t];
+      xs[i * 64 + t] = xs[p * 64 + t];
+      xs[p * 64 + t] = tmp;
+    }
+  }
+  for (int i = 0; i < n; ++i) {
+    T xi = xs[i * 64 + t];
+    for (int k = 0; k < i; ++k) {
+      const T prod = lu[(int64_t)i * lda + k] * xs[k * 64 + t];
+      xi = xi - prod;
+    }
+    xs[i * 64 + t] = xi;
+  }
+  for (int i = n - 1; i >= 0; --i) {
+    T xi = xs[i * 64 + t];
+    for (int k = i + 1; k < n; ++k) {
+      const T prod = lu[(int64_t)i * lda + k] * xs[k * 64 + t];
+      xi = xi - prod;
+    }
+    xs[i * 64 + t] = xi / lu[(int64_t)i * lda + i];
+  }
+  for (int i = 0; i < n; ++i) b[(int64_t)i * ldb + c] = xs[i * 64 + t];
+}
+
+// Right-hand sides up to which a wave each wins: its workgroups hold eight and
+// a copy of the factors, so beyond they come in rounds.  A call, us, a wave / a
+// thread each: FP64 n=128 340 / 374 at 4096, 480 / 376 at 5000, n=32 77 / 80 and
+// 88 / 81; FP32 n=128 332 / 343 at 8192, 402 / 345 at 10000, n=16 54 / 57 at 4096,
+// 62 / 57 at 8192.
+template <typename T>
+static int exact_wave_rhs(int n) {
+  return sizeof(T) == 4 && n > 32 ? 8192 : 4096;
+}
 template <typename T>
 hipError_t launch_getrs_exact(lair_context *ctx, int n, int nrhs, const T *lu, int64_t lda,
                               const int64_t *ipiv, T *b, int64_t ldb) {
   if (n <= 0 || nrhs <= 0) return hipSuccess;
   if (n > kExactOrderMax) return hipErrorInvalidValue;
+  if (nrhs > exact_wave_rhs<T>(n)) {
+    const int slot = prof_begin(ctx, LAIR_KCLASS_GETRS);
+    getrs_exact_many_kernel<T><<<(nrhs + 63) / 64, 64, sizeof(T) * 64 * (size_t)n, ctx->stream>>>(n, nrhs, lu, lda, ipiv,
+                                                                                              b, ldb, ctx->err);
+    prof_end(ctx, slot, LAIR_KCLASS_GETRS, 2.0 * n * n * nrhs);
+    return hipGetLastError();
+  }
   const int nw = std::min(nrhs, kExactWaves);
   const size_t shm = sizeof(T) * ((size_t)nw * 2 * kExactPad + (size_t)n * (n | 1));
   static bool once = ((void)hipFuncSetAttribute(reinterpret_cast<const void *>(getrs_exact_kernel<T>),

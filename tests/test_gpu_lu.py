@@ -358,3 +358,28 @@ def test_sgetrs_many_rhs(n, nrhs):
     assert berr <= 8 * n * eps32
     x1 = L.getrs(g, piv, b[:, 5])
     assert np.abs(x1 - x[:, 5]).max() <= 64 * n * eps32 * np.abs(x1).max()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [1, 7, 64, 128])
+def test_small_getrs_operation_order_any_nrhs(n, dtype):
+    """n <= 128: every right-hand side takes the reference's operations in its
+    order (getrs.rs:23-36), with a wave per right-hand side or, beyond 4096 of
+    them (FP32, n > 32: 8192), a thread."""
+    lim = 8192 if dtype == np.float32 and n > 32 else 4096
+    a = inputs.gaussian_matrix(71 + n, n, n).astype(dtype)
+    lu = a.copy()
+    piv, _ = (O.getrf if dtype == np.float64 else O.sgetrf)(lu)
+    b = inputs.gaussian_matrix(72 + n, n, lim + 1).astype(dtype)
+    x = b.copy()
+    for i, p in enumerate(piv):
+        x[[i, p]] = x[[p, i]]
+    for i in range(n):
+        for k in range(i):
+            x[i] -= lu[i, k] * x[k]
+    for i in range(n - 1, -1, -1):
+        for k in range(i + 1, n):
+            x[i] -= lu[i, k] * x[k]
+        x[i] /= lu[i, i]
+    for r in (1, 9, lim, lim + 1):
+        assert np.array_equal(L.getrs(lu, piv, np.ascontiguousarray(b[:, :r])), x[:, :r]), r
