@@ -323,8 +323,11 @@ hipError_t launch_cgetrs(lair_context *ctx, int n, int nrhs, const T *lu, int64_
              (double)sizeof(T) * ((double)n * n * nrhs + 2.0 * n * nrhs));
     return hipGetLastError();
   }
-  // Passes of at most 64 right-hand sides bound the workspaces.
-  const int chunk = std::min(nrhs, 64);
+  // Passes of as many right-hand sides as the workspaces hold: 64 of the
+  // largest order (50 MB with f64 components), more of smaller ones, so that a
+  // small system with many of them still fills the chip (n=150 with 300, f64
+  // components: 171 us in one workgroup per right-hand side, 265 in passes of 64).
+  const int chunk = std::min(nrhs, 64 * kComplexGetrsMax / n);
   hipError_t e = ensure(ctx->ws_tmp2, sizeof(T) * (size_t)n * chunk);
   if (e != hipSuccess) return e;
   CflowArgs<T> a;

@@ -61,3 +61,17 @@ def test_complex_getrs_waits_give_up(n, nrhs, dtype):
     for d in (dlu, dp, db):
         d.free()
     ctx.close()
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+def test_complex_getrs_more_than_one_pass(dtype):
+    """n=150: a pass takes 64 * 16384 / 150 = 6990 right-hand sides; the last
+    ones come in a second pass.  The same right-hand sides alone (a pass of
+    their own) give the same bits."""
+    n, nrhs = 150, 6993
+    a = (inputs.gaussian_matrix(8500, n, n) + 4.0 * np.sqrt(n) * np.eye(n)).astype(dtype)
+    b = (inputs.gaussian_matrix(8501, n, nrhs) + 1j * inputs.gaussian_matrix(8502, n, nrhs)).astype(dtype)
+    piv, _ = L.getrf(a)
+    x = L.getrs(a, piv, b)
+    for c in (0, 6989, 6990, 6992):
+        assert np.array_equal(L.getrs(a, piv, b[:, c:c + 1].copy()), x[:, c:c + 1]), c
