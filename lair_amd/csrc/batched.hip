@@ -185,10 +185,11 @@ struct BatchSolver {
   const int n, r;
   const BatchBuf<T> A, B;
   int sing;
+  unsigned none;  // columns of the block without a candidate
 
   __device__ __forceinline__ BatchSolver(Lds &s, int n_, int r_, T *a, T *b)
       : S(s), t(threadIdx.x), lane(threadIdx.x & 63), wave(threadIdx.x >> 6), g(lane >> 4), lc(lane & 15), n(n_),
-        r(r_), A(a, n_ * n_), B(b, n_ * r_), sing(-1) {}
+        r(r_), A(a, n_ * n_), B(b, n_ * r_), sing(-1), none(0) {}
 
   // Barrier for data in LDS only: unlike __syncthreads it does not wait for
   // global loads and stores in flight.
@@ -287,7 +288,7 @@ struct BatchSolver {
         }
         const bool singular = bk == 0;
         pr = singular ? d : pr;
-        sing = singular ? kb + d : sing;
+        none = singular ? none | 1u << d : none;
         pos = pos == d ? pr : (pos == pr ? d : pos);
         S.piv[kb + d] = (unsigned char)(kb + pr);
         if (__builtin_expect(!singular && pos > d, 1)) {
@@ -325,6 +326,14 @@ struct BatchSolver {
     return c;
   }
 
+  // 0, or NaN if an entry is not finite.
+  __device__ __forceinline__ static T zero_if_finite(v4 x) {
+    T s = T(0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s = __builtin_elementwise_fma(x[e], T(0), s);
+    return s;
+  }
+
   // Inverse of unit lower triangle h of the block's diagonal: lane j column
   // j, by substitution.  Rows past the matrix are zero.
   __device__ __forceinline__ void invert(int h) {
@@ -343,13 +352,93 @@ struct BatchSolver {
     }
   }
 
+  // Products with an inverted triangle and with whole rows of L multiply every
+  // row of a column with every other: they make NaN of rows that an infinity, a
+  // NaN or a column without a candidate (which eliminates nothing,
+  // getrf.rs:72-73) does not reach.  Where there is one, the elimination goes by
+  // substitution, a column of L after the other.  Looking for them costs 1 - 2 %
+  // (5000 systems of n = 8 .. 256: FP64 2.06 against 2.08 ms, FP32 1.25 against
+  // 1.27).  The right panel, in LDS, a row per thread:
+  __device__ __forceinline__ void right_panel_any(int rows) {
+#pragma clang fp contract(off)
+#pragma unroll 1
+    for (int j = 0; j < H; ++j) {
+      if (!(none >> j & 1u) && t > j && t < rows) {
+        const T l = S.p[t][j];
+#pragma unroll 1
+        for (int c = H; c < W; ++c) {
+          const T e = l * S.p[j][c];
+          S.p[t][c] = S.p[t][c] - e;
+        }
+      }
+      lds_sync();
+    }
+  }
+  // A chunk (see chunk), in memory, four rows at a time, without the columns of
+  // L in `skip` (right-hand sides take L as it is stored, getrs.rs:25-29).
+  // (Rolled: it shares the registers of the loop that it stands in.)
+  __device__ __forceinline__ void chunk_any(const BatchBuf<T> &q, uint32_t ld, uint32_t col, int kb, int w,
+                                            unsigned skip) {
+#pragma clang fp contract(off)
+    const int rows = n - kb, cnt = S.cnt;
+    const uint32_t base = kb * ld + col;
+    T u[W / 4], val[W / 4];
+#pragma unroll
+    for (int e = 0; e < W / 4; ++e) {
+      u[e] = q.load(base + S.src[4 * e + g] * ld);
+      val[e] = q.load(base + S.from[max(min(4 * e + g, cnt - 1), 0)] * ld);
+    }
+#pragma unroll
+    for (int e = 0; e < W / 4; ++e) {
+      q.store(base + (4 * e + g) * ld, u[e]);
+      if (4 * e + g < cnt) q.store(base + S.rows[4 * e + g] * ld, val[e]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    // Rows of the block: column k of L11 after the others.
+#pragma unroll 1
+    for (int k = 0; k + 1 < w; ++k) {
+      if (!(skip >> k & 1u)) {
+        const T uk = q.load(base + k * ld);
+#pragma unroll 1
+        for (int i = k + 1 + g; i < w; i += 4) {
+          const T e = S.p[i][k] * uk;
+          q.store(base + i * ld, q.load(base + i * ld) - e);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+      }
+    }
+    // Rows below.
+#pragma unroll 1
+    for (int i = W + g; i < rows; i += 4) {
+      T x = q.load(base + i * ld);
+#pragma unroll 1
+      for (int k0 = 0; k0 < W; k0 += 8) {
+        T uk[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) uk[k] = q.load(base + (k0 + k) * ld);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const T e = S.p[i][k0 + k] * uk[k];
+          x = skip >> (k0 + k) & 1u ? x : x - e;
+        }
+      }
+      q.store(base + i * ld, x);
+    }
+  }
+
   // The left panel's elimination applied to the right panel, in LDS.
   __device__ __forceinline__ void right_panel(int rows) {
     v4 u;
 #pragma unroll
     for (int e = 0; e < 4; ++e) u[e] = S.p[M::row(g, e)][H + lc];
     u = prod(&S.inv[0][lc][0], u);
+    // (The same in every wave.)
+    const bool odd = none != 0 || !__all(zero_if_finite(u) == T(0));
     lds_sync();
+    if (__builtin_expect(odd, 0)) {
+      right_panel_any(rows);
+      return;
+    }
     if (wave == 0) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) S.p[M::row(g, e)][H + lc] = u[e];
@@ -367,12 +456,14 @@ struct BatchSolver {
     const int c0 = kb + w, na = (n - c0 + 15) / 16;  // chunks of A, then one of B
     for (int ch = wave; ch <= na; ch += NW) {
       const int c = ch < na ? c0 + 16 * ch + lc : lc, ld = ch < na ? n : r;
-      chunk(ch < na ? A : B, ld, c < ld ? c : A.kNone / 2, kb, w);
+      const uint32_t col = c < ld ? c : A.kNone / 2;
+      if (!chunk(ch < na ? A : B, ld, col, kb, w)) chunk_any(ch < na ? A : B, ld, col, kb, w, ch < na ? none : 0);
     }
   }
 
-  // One chunk: lane column `col` of the row-major q with rows of ld.
-  __device__ __forceinline__ void chunk(const BatchBuf<T> &q, uint32_t ld, uint32_t col, int kb, int w) {
+  // One chunk: lane column `col` of the row-major q with rows of ld.  False,
+  // and nothing done, where it is for chunk_any.
+  __device__ __forceinline__ bool chunk(const BatchBuf<T> &q, uint32_t ld, uint32_t col, int kb, int w) {
     const int rows = n - kb, cnt = S.cnt;
     const uint32_t base = kb * ld + col, lrow0 = base + M::row(g, 0) * ld;
     constexpr int RS = M::kStep;
@@ -391,17 +482,26 @@ struct BatchSolver {
       u1[e] = q.load(base + S.src[M::row(g, e) + H] * ld);
     }
     // Rows below the block that receive another row.
+    T val[W / 4];
     if (cnt) {
-      T val[W / 4];
 #pragma unroll
       for (int e = 0; e < W / 4; ++e) val[e] = q.load(base + S.from[min(4 * e + g, cnt - 1)] * ld);
+    } else if (rows > W) {
+      load(W, cur);
+    }
+    // Where it is for chunk_any every store goes past the end (a branch here
+    // cost the registers of the loop below).
+    const bool odd = none != 0 || !__all(zero_if_finite(u0) + zero_if_finite(u1) == T(0));
+    const uint32_t off = odd ? q.kNone / 2 : 0;
+    const uint32_t srow0 = lrow0 + off;
+    if (cnt) {
 #pragma unroll
       for (int e = 0; e < W / 4; ++e)
-        if (4 * e + g < cnt) q.store(base + S.rows[4 * e + g] * ld, val[e]);
+        if (4 * e + g < cnt) q.store(base + off + S.rows[4 * e + g] * ld, val[e]);
       // The tiles below are read with another lane layout.
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+      if (rows > W) load(W, cur);
     }
-    if (rows > W) load(W, cur);
     u0 = prod(&S.inv[0][lc][0], u0);
     if (w > H) {
       u1 -= prod(&S.p[H + lc][0], u0);
@@ -409,8 +509,8 @@ struct BatchSolver {
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      q.store(lrow0 + RS * e * ld, u0[e]);
-      if (w > H) q.store(lrow0 + (H + RS * e) * ld, u1[e]);
+      q.store(srow0 + RS * e * ld, u0[e]);
+      if (w > H) q.store(srow0 + (H + RS * e) * ld, u1[e]);
     }
     for (int i0 = W; i0 < rows; i0 += 64) {
       v4 nxt[4];
@@ -421,12 +521,13 @@ struct BatchSolver {
           const T *lrow = &S.p[i0 + 16 * b + lc][0];
           cur[b] -= prod(lrow, u0) + prod(lrow + H, u1);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) q.store(lrow0 + (i0 + 16 * b + RS * e) * ld, cur[b][e]);
+          for (int e = 0; e < 4; ++e) q.store(srow0 + (i0 + 16 * b + RS * e) * ld, cur[b][e]);
         }
       }
 #pragma unroll
       for (int b = 0; b < 4; ++b) cur[b] = nxt[b];
     }
+    return !odd;
   }
 
   __device__ __forceinline__ void factor() {
@@ -444,6 +545,7 @@ struct BatchSolver {
         for (int e = 0; e < W; ++e) S.p[tr + RP * e][tc] = x[e];
       }
       if (t == 0) S.cnt = 0;
+      none = 0;
       lds_sync();
       int org = t;
       for (int half = 0;; ++half) {
@@ -451,6 +553,7 @@ struct BatchSolver {
         int pos = t;
         get(v, &S.p[t][half * H]);
         panel(v, pos, kb, half * H, w);
+        none = (unsigned)__builtin_amdgcn_readfirstlane((int)none);
         place(v, pos, half, org);
         if (wave == 0) invert(half);
         if (half == 1 || w <= H) break;
@@ -462,6 +565,7 @@ struct BatchSolver {
 #pragma unroll
       for (int e = 0; e < W; ++e) A.store(at + RP * e * n, S.p[tr + RP * e][tc]);
       lds_sync();
+      if (none != 0) sing = kb + 31 - __builtin_clz(none);
       if (has) {
         S.orig[kb + t] = (unsigned char)o;
         S.hist[blk][o] = (unsigned char)(kb + t);

@@ -97,3 +97,57 @@ def test_ties_and_zero_columns(dtype):
         _, piv_o, sing_o = _oracle(A)
         np.testing.assert_array_equal(piv, piv_o, err_msg=f"{i} n={len(A)}")
         assert info == sing_o
+
+
+def _substitute(lu, piv, B):
+    """getrs.rs:23-36 in the matrix's own type."""
+    x, n = B.copy(), len(lu)
+    for i, p in enumerate(piv):
+        x[[i, p]] = x[[p, i]]
+    with np.errstate(all="ignore"):
+        for k in range(n):
+            x[k + 1:] -= lu[k + 1:, k:k + 1] * x[k]
+        for i in range(n - 1, -1, -1):
+            for k in range(i + 1, n):
+                x[i] -= lu[i, k] * x[k]
+            x[i] /= lu[i, i]
+    return x
+
+
+def _same_classes(got, ref, msg):
+    for f in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(f(got), f(ref), err_msg=f"{msg} {f.__name__}")
+
+
+NONFINITE = [20, 40, 64, 100, 128, 200, 256]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["inf", "inf_late", "nan_column", "zero_column"])
+def test_nonfinite_entries(kind, dtype):
+    """An infinity in a column right of its block, and columns of zeros or NaN
+    (which eliminate nothing) whose pivot row holds one: pivots, info, and which
+    entries of LU and X are NaN, +inf and -inf are those of the column by column
+    elimination."""
+    rng = np.random.default_rng(61)
+    As, Bs = [], []
+    for n in NONFINITE:
+        A = rng.standard_normal((n, n)).astype(dtype) + n * np.eye(n, dtype=dtype)
+        c = n // 3
+        if kind == "inf":
+            A[5, n - 4] = np.inf
+        elif kind == "inf_late":
+            A[n - 3, n - 2] = -np.inf
+        else:
+            for c in (1, n // 3):
+                A[:, c] = 0.0 if kind == "zero_column" else np.nan
+                A[c, n - 2] = np.inf
+        As.append(A)
+        Bs.append(rng.standard_normal((n, 3)).astype(dtype))
+    for A, B, (lu, x, piv, info) in zip(As, Bs, _run(As, Bs, dtype)):
+        ref, piv_o, sing_o = _oracle(A)
+        msg = f"{kind} n={len(A)}"
+        np.testing.assert_array_equal(piv, piv_o, err_msg=msg)
+        assert info == sing_o, msg
+        _same_classes(lu, ref, msg)
+        _same_classes(x, _substitute(ref, piv_o, B), msg)
