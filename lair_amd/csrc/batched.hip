@@ -606,7 +606,9 @@ struct BatchSolver {
   // lanes holds row lc of the block (u, its diagonal d) and of one right-hand
   // side (x); returns that row of the solution.  The quotient comes from the
   // reciprocal rd and one correction by its remainder, which gives the rounded
-  // quotient itself for a d far from the ends of the exponent range.
+  // quotient itself while d, x and the quotient are clear of the subnormal range,
+  // and about one unit in the last place (of the subnormals, there) otherwise.
+  // The caller looks at the range of d and at the results.
   template <int I = H - 1>
   __device__ __forceinline__ void tri(const T (&u)[H], T d, T rd, int w, T x, T &out) const {
     if (__builtin_expect(I < w, 1)) {
@@ -617,7 +619,7 @@ struct BatchSolver {
     }
     if constexpr (I > 0) tri<I - 1>(u, d, rd, w, x, out);
   }
-  // The same with the division itself, for any d (rolled: rarely taken).
+  // The same with the division itself, for any d and x (rolled: rarely taken).
   __device__ __noinline__ static T tri_any(BatchBuf<T> a, int n, int kb, int w, T d, T x) {
     const int l = threadIdx.x & 15;
     T out = T(0);
@@ -662,10 +664,9 @@ struct BatchSolver {
           const int c = min(c0 + g, r - 1);
           const T x = sY[c * YP + kb + min(lc, w - 1)];
           T out = T(0);
-          if (__builtin_expect(fast, 1))
-            tri(ud, d, rd, w, x, out);
-          else
-            out = tri_any(A, n, kb, w, d, x);
+          if (__builtin_expect(fast, 1)) tri(ud, d, rd, w, x, out);
+          // (x infinite, or a quotient out of range: the remainder is NaN.)
+          if (__builtin_expect(!fast || !__all(out - out == T(0)), 0)) out = tri_any(A, n, kb, w, d, x);
           if (c0 + g < r && lc < w) sY[c * YP + kb + lc] = out;
         }
       }

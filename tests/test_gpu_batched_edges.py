@@ -151,3 +151,39 @@ def test_nonfinite_entries(kind, dtype):
         assert info == sing_o, msg
         _same_classes(lu, ref, msg)
         _same_classes(x, _substitute(ref, piv_o, B), msg)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["rhs_inf", "rhs_inf_first", "overflow", "zero_pivot"])
+def test_quotients_out_of_range(kind, dtype):
+    """Infinite right-hand sides, quotients that overflow and a zero pivot: the
+    back substitution's results are those of divisions."""
+    rng = np.random.default_rng(62)
+    As, Bs = [], []
+    big = dtype(np.finfo(dtype).max / 4)
+    for n in NONFINITE:
+        A = rng.standard_normal((n, n)).astype(dtype) + n * np.eye(n, dtype=dtype)
+        B = rng.standard_normal((n, 3)).astype(dtype)
+        if kind == "rhs_inf":
+            B[n - 2, 1] = np.inf
+        elif kind == "rhs_inf_first":
+            B[0, 2] = -np.inf
+        elif kind == "overflow":
+            A = (0.03 * np.eye(n)).astype(dtype)
+            A[0, 1:] = dtype(0.01)
+            B[0, 1] = big
+            B[0, 0] = -big
+        else:
+            A = np.triu(A)
+            A[n // 2, n // 2] = 0.0
+        As.append(A)
+        Bs.append(B)
+    for A, B, (lu, x, piv, info) in zip(As, Bs, _run(As, Bs, dtype)):
+        ref, piv_o, sing_o = _oracle(A)
+        msg = f"{kind} n={len(A)}"
+        np.testing.assert_array_equal(piv, piv_o, err_msg=msg)
+        assert info == sing_o, msg
+        want = _substitute(ref, piv_o, B)
+        assert not np.isfinite(want).all()
+        _same_classes(lu, ref, msg)
+        _same_classes(x, want, msg)
