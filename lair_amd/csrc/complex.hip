@@ -166,7 +166,9 @@ __device__ __forceinline__ cplx<R> csel(bool c, cplx<R> a, cplx<R> b) {
 // The quotients of the back substitution are x conj(d) / |d|^2 by the
 // precomputed inverse of d and one correction by the remainder, which is at
 // least as close as the direct formula; blocks with a diagonal entry far from
-// 1 in the exponent use the direct formula.
+// 1 in the exponent use the direct formula, and so does a block again whose
+// result is not finite (an infinite right-hand side, or a quotient that
+// overflows, makes NaN of the remainder).
 //
 // Bound by the chain: 64 substitution steps per block (1.4 us with f64
 // components, 5.5 us with the quotients) and one round trip of the words.
@@ -279,27 +281,32 @@ __global__ void __launch_bounds__(256, 2) cgetrs_flow_kernel(CflowArgs<T> p) {
     const T dg = dt[lane * LD + lane];
     const R ns = dg.re * dg.re + dg.im * dg.im;
     const R lo = sizeof(R) == 8 ? R(0x1p-500) : R(0x1p-60f), hi = sizeof(R) == 8 ? R(0x1p500) : R(0x1p60f);
-    const bool fast = __all(lane >= w || (ns >= lo && ns <= hi));
+    bool fast = __all(lane >= w || (ns >= lo && ns <= hi));
     const T inv(dg.re / ns, -dg.im / ns);
-    for (int k0 = (w - 1) / 8 * 8; k0 >= 0; k0 -= 8) {
-      T u[8];
+    for (;;) {
+      for (int k0 = (w - 1) / 8 * 8; k0 >= 0; k0 -= 8) {
+        T u[8];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) u[q] = dt[(k0 + q) * LD + lane];
+        for (int q = 0; q < 8; ++q) u[q] = dt[(k0 + q) * LD + lane];
 #pragma unroll
-      for (int q = 7; q >= 0; --q) {
-        if (k0 + q < w) {
-          T v;
-          if (fast) {
-            v = csub_mul(T(0), T(-x.re, -x.im), inv);
-            v = csub_mul(v, T(0) - csub_mul(x, v, dg), inv);
-          } else {
-            v = cplx_div(x, dg);
+        for (int q = 7; q >= 0; --q) {
+          if (k0 + q < w) {
+            T v;
+            if (fast) {
+              v = csub_mul(T(0), T(-x.re, -x.im), inv);
+              v = csub_mul(v, T(0) - csub_mul(x, v, dg), inv);
+            } else {
+              v = cplx_div(x, dg);
+            }
+            x = csel(lane == k0 + q, v, x);
+            const T nx = csub_mul(x, u[q], readlane_t(x, k0 + q));
+            x = csel(lane < k0 + q, nx, x);
           }
-          x = csel(lane == k0 + q, v, x);
-          const T nx = csub_mul(x, u[q], readlane_t(x, k0 + q));
-          x = csel(lane < k0 + q, nx, x);
         }
       }
+      if (!fast || __all(lane >= w || (x.re - x.re == R(0) && x.im - x.im == R(0)))) break;
+      fast = false;
+      x = ys[lane];
     }
   }
   if (lane < w) {

@@ -75,3 +75,39 @@ def test_complex_getrs_more_than_one_pass(dtype):
     x = L.getrs(a, piv, b)
     for c in (0, 6989, 6990, 6992):
         assert np.array_equal(L.getrs(a, piv, b[:, c:c + 1].copy()), x[:, c:c + 1]), c
+
+
+def _back_substitute(u, b):
+    """x with u x = b, component by component: num-complex's product and quotient."""
+    x, n = b.copy(), len(b)
+    with np.errstate(all="ignore"):
+        for i in range(n - 1, -1, -1):
+            for k in range(i + 1, n):
+                re = u[i, k].real * x[k].real - u[i, k].imag * x[k].imag
+                im = u[i, k].real * x[k].imag + u[i, k].imag * x[k].real
+                x.real[i] -= re
+                x.imag[i] -= im
+            d = u[i, i]
+            ns = d.real * d.real + d.imag * d.imag
+            re = (x[i].real * d.real + x[i].imag * d.imag) / ns
+            im = (x[i].imag * d.real - x[i].real * d.imag) / ns
+            x.real[i], x.imag[i] = re, im
+    return x
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("n", [130, 192, 300])
+def test_complex_quotients_that_overflow(n, dtype):
+    """A quotient that overflows is infinite, not NaN, and the rows above see
+    it so: the same entries are NaN, +inf and -inf as with plain quotients."""
+    big = np.finfo(dtype).max / 4
+    u = (np.triu(np.full((n, n), 0.01)) + 0.03 * np.eye(n)).astype(dtype)
+    b = (inputs.gaussian_matrix(8600, n, 3) + 1j * inputs.gaussian_matrix(8601, n, 3)).astype(dtype)
+    b[0, 1] = big
+    b[70, 2] = -1j * big
+    want = _back_substitute(u, b)
+    got = L.getrs(u, np.arange(n), b)
+    assert np.isposinf(want[0, 1].real) and np.isfinite(want[:, 0]).all()
+    for part in ("real", "imag"):
+        for f in (np.isnan, np.isposinf, np.isneginf):
+            np.testing.assert_array_equal(f(getattr(got, part)), f(getattr(want, part)), err_msg=f"{part} {f.__name__}")
