@@ -26,12 +26,12 @@
 //
 // Bound by the chain of columns (850 cycles with one wave, 1400 with four) at
 // 2 to 7 workgroups per CU and, for large n, by the latency of the passes over
-// the trailing matrix; the code (37 - 45 KB) has to stay within the 64 KB
+// the trailing matrix; the code (40 - 51 KB) has to stay within the 64 KB
 // instruction cache (at 61 - 71 KB a column took twice as long).  Whole
 // solves, input copies included, against one persistent kernel with panels of
 // 8 or 16 columns and register-tile updates chosen by timing: 4096 systems in
-// FP64 of n = 256: 4.82 ms against 10.91; 128: 1.15 against 2.42; 64: 0.25
-// against 0.70; 32: 0.11 against 0.33; 5000 of n = 8 .. 256: 2.47 against 4.74;
+// FP64 of n = 256: 4.80 ms against 10.66; 128: 1.16 against 2.38; 64: 0.27
+// against 0.71; 32: 0.13 against 0.34; 5000 of n = 8 .. 256: 2.49 against 4.78;
 // 3000 in FP32 of n = 8 .. 128: 0.23 against 0.48.
 #include <algorithm>
 #include <climits>

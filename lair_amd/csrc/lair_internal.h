@@ -57,9 +57,9 @@ constexpr int kRpRowWords = 256;  // >= leaf width * 32-bit words per element
 constexpr size_t kRpBlkOff = 2 * (size_t)kMaxPanelWG * kRpRecWords;
 constexpr size_t kRpMvOff = kRpBlkOff + 2 * (size_t)kRpMaxW * kRpRowWords;
 constexpr size_t kRpBufWords = kRpMvOff + 2 * (size_t)kRpMaxCols * kRpRowWords;
-// Widest complex panel (the triangular solve with L11 keeps L11 in LDS),
-// and the largest order of the complex getrs (unknowns of a right-hand side
-// held in registers of one 1024-thread workgroup, 16 per thread).
+// Widest complex panel (the triangular solve with L11 keeps L11 in LDS), and
+// the largest order of the complex getrs (the limit its entry points state; it
+// also sizes the workspaces of a pass of right-hand sides).
 constexpr int kComplexMaxNb = 64;
 constexpr int kComplexGetrsMax = 16384;
 
@@ -325,7 +325,7 @@ hipError_t launch_dgemm_splitk_store(lair_context *ctx, int M, int N, int K, int
 hipError_t launch_bgemm_tile(lair_context *ctx, int ns, int M, int N, int K, const float *A,
                              int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc);
 
-// Persistent batched solver (batched.hip): device metadata and launch shape.
+// Batched solver (batched.hip): device metadata of one size class.
 struct BatchLaunch {
   int count = 0;
   int nmax = 0;           // largest order of the launch

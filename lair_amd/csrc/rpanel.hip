@@ -24,8 +24,9 @@
 //    are exchanged (one round trip per W columns), every workgroup solves
 //    U = L11^-1 A for them and updates its own rows with rank W, in place in
 //    global memory (its XCD's L2), with the same operations in the same order
-//    as the unblocked loop: a leaf's factors do not depend on W or P.  With
-//    P > 1 only the next sub-panel's columns are updated at once; the rest
+//    as the unblocked loop: a leaf's factors do not depend on W or P.  (A
+//    column without a candidate eliminates nothing; the sub-panel keeps a mask
+//    of them.)  With P > 1 only the next sub-panel's columns are updated at once; the rest
 //    fills the waits of the next column loop.
 //
 // Measured per leaf, against a leaf that kept 256 rows per workgroup in LDS
@@ -33,7 +34,8 @@
 // FP64, 64 columns: 70 against 165 us at 100 rows, 104 / 172 at 512, 152 /
 // 185 at 1024, 182 / 190 at 2048 inside a factorization; FP32, 128 columns:
 // 211 / 370 us at 512 rows, 346 / 385 at 1024, 369 / 397 at 4096, 411 / 435
-// at 16384.  A column costs about 0.9 us of instructions and LDS latencies
+// at 16384; complex<f64>, 64 columns of 3000 rows, call included: 303 / 402.  A
+// column costs about 0.9 us of instructions and LDS latencies (complex: 1.6)
 // and, with P > 1, 0.8 us of round trip and 0.6 us for the slowest of the
 // others.
 //
@@ -175,14 +177,6 @@ __device__ __forceinline__ void pin(T &x) {
   } else {
     __asm__ volatile("" : "+v"(x));
   }
-}
-
-template <typename T>
-__device__ __forceinline__ T sel(bool c, T x, T y) {
-  if constexpr (cplx_traits<T>::is)
-    return T(c ? x.re : y.re, c ? x.im : y.im);
-  else
-    return c ? x : y;
 }
 
 // N elements from 16-byte aligned LDS, by 16-byte reads.

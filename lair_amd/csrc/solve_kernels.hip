@@ -1244,9 +1244,10 @@ __global__ void __launch_bounds__(256) trsv_ir_kernel(TrsvArgs<float> p, IrFuse 
 //    as the second operand of x = D y.
 // Bound by the chain of blocks: one round trip of the words (0.8 us), the
 // products with the last block and with D (0.4 us each in FP64) and their
-// barriers: 3.2 us per block in FP64.  Both solves of n = 4096 with 64
-// right-hand sides: 0.50 ms, where the vector kernel took 1.88 ms (14.7 us
-// per block); with 16: 0.42 ms against 1.03.
+// barriers: 3.7 us per block in FP64 (236 us a solve of n = 4096), 7.2 us per
+// block of 128 rows in FP32.  Both solves of n = 4096 with 64 right-hand sides,
+// call included: 0.50 ms, where the vector kernel took 1.88 ms (14.7 us per
+// block); with 16: 0.42 ms against 1.03.
 template <typename T>
 struct TrsmMfma;
 template <>

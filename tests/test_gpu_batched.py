@@ -1,5 +1,5 @@
-"""Batched uneven solves (one persistent, graph-captured launch) against the
-CPU oracle: per system, pivots bit-exact with the reference's row-major LU
+"""Batched uneven solves (one captured graph with a launch per size class)
+against the CPU oracle: per system, pivots bit-exact with the reference's row-major LU
 (src/lapack/getrf.rs:46-120) and backward error of X <= n * eps of the
 arithmetic; graph replays reproduce the eager result bit for bit."""
 import numpy as np
@@ -60,9 +60,8 @@ def ctx():
     c.close()
 
 
-# Without the autotuner the plan keeps its first candidate: 16-column panels
-# with every system updated in global memory; the autotuned plans of these
-# batches stage the smaller systems in LDS.
+# The autotune flag is accepted and changes nothing: 16-column register panels,
+# every system updated in global memory.
 @pytest.mark.parametrize("autotune", [True, False])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_batched_matches_oracle(ctx, dtype, autotune):

@@ -187,3 +187,22 @@ def test_quotients_out_of_range(kind, dtype):
         assert not np.isfinite(want).all()
         _same_classes(lu, ref, msg)
         _same_classes(x, want, msg)
+
+
+def test_config_of_the_largest_class():
+    """The plan's launch shape is that of its largest systems' class: a
+    workgroup for each of them."""
+    rng = np.random.default_rng(63)
+    ctx = L.Context()
+    for ns, grid in (([40, 64, 65, 128, 129, 256, 200], 3), ([8, 128, 65, 64], 2), ([64, 1, 33], 3)):
+        ns = np.array(ns, np.int32)
+        rs = np.ones(len(ns), np.int32)
+        da = L.DeviceArray.from_host(rng.standard_normal((int((ns * ns).sum()), 1)))
+        db = L.DeviceArray.from_host(rng.standard_normal((int(ns.sum()), 1)))
+        dp, di = L.DeviceArray(int(ns.sum()), 1, np.int64), L.DeviceArray(len(ns), 1, np.int32)
+        plan = L.BatchedPlan(ctx, ns, rs, da, db, dp, di)
+        assert plan.config()["grid"] == grid
+        plan.close()
+        for d in (da, db, dp, di):
+            d.free()
+    ctx.close()

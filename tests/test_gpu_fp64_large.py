@@ -1,6 +1,5 @@
-"""FP64 LU at an order where the first panels use the narrow resident leaves
-(32 columns and 512 rows per workgroup while at least 12288 rows remain,
-then 64 columns): the getrf.rs:46-120 elimination with the panel -> laswp ->
+"""FP64 LU at an order whose panels hold two leaves of 64 columns each, over up
+to 26 workgroups of 512 rows: the getrf.rs:46-120 elimination with the panel -> laswp ->
 trsm -> gemm blocking of getrf.rs:216-322.
 
 Checked on the host, O(n^2):
